@@ -153,6 +153,61 @@ def test_fused_small_route_segment_bit_exact(T, E, K, NS, mode):
     assert int(seg.n_tiles.item()) == ets[-1]
 
 
+@pytest.mark.parametrize("T,K,E,NS", [(64, 16, 1024, 0), (93, 10, 512, 1), (341, 3, 2047, 0),
+                                      (1, 1, 1, 0), (205, 4, 6, 1)])
+def test_small_segmentation_table_edges(T, K, E, NS):
+    """The ballot ranks of 1023, 1024 and 1025 pairs, wide and narrow bucket
+    tables, one pair, and buckets whose rows spread over many waves."""
+    ids, wts = random_routing(T, K, E, seed=T, invalid_frac=0.1, zero_frac=0.1)
+    seg = L.segmentation(T, K, E, NS, 128, torch.device("cuda"))
+    if seg.small and E <= 1024:
+        seg.run_small(2, torch.from_numpy(ids).cuda(), torch.from_numpy(wts).cuda(),
+                      drop_zero=True)
+        torch.cuda.synchronize()
+    else:   # past the one-launch envelope
+        seg = _gpu_segment(ids, wts, E, NS, True)
+    ref = oracle.segment(ids, wts, E, NS, True)
+    np.testing.assert_array_equal(seg.seg_start.cpu().numpy(), ref["seg_start"])
+    for k in ("sorted_pair", "sorted_tok", "inv"):
+        np.testing.assert_array_equal(getattr(seg, k).cpu().numpy()[: seg.A], ref[k])
+
+
+@pytest.mark.parametrize("T,E,K,mode", [(8, 256, 8, 1), (15, 256, 8, 1), (16, 512, 10, 0),
+                                        (7, 512, 10, 0)])
+def test_wave_routed_small_batch_bit_exact(T, E, K, mode):
+    """More than 64 pairs, at most 16 tokens: one routing wave per token."""
+    rng = np.random.default_rng(T + E)
+    logits = rng.standard_normal((T, E)).astype(np.float32)
+    logits[1::2, : E // 2] = np.round(logits[1::2, : E // 2] * 2) / 2   # ties
+    dev = torch.device("cuda")
+    seg = L.segmentation(T, K, E, 1, 16, dev)
+    ids = torch.empty((T, K), dtype=torch.int32, device=dev)
+    wts = torch.empty((T, K), dtype=torch.float32, device=dev)
+    kw = dict(n_group=8, topk_group=4, routed_scaling=2.5) if mode == 1 else {}
+    seg.run_small(mode, ids, wts, logits=torch.from_numpy(logits).to(dev), **kw)
+    torch.cuda.synchronize()
+    rids, rwts = (oracle.route_grouped_sigmoid(logits, None, 8, 4, K, 2.5) if mode == 1
+                  else oracle.route_softmax_topk(logits, K))
+    np.testing.assert_array_equal(ids.cpu().numpy(), rids)
+    np.testing.assert_array_equal(wts.cpu().numpy().view(np.uint32), rwts.view(np.uint32))
+    ref = oracle.segment(rids, rwts, E, 1, True)
+    np.testing.assert_array_equal(seg.seg_start.cpu().numpy(), ref["seg_start"])
+    np.testing.assert_array_equal(seg.sorted_pair.cpu().numpy()[: seg.A], ref["sorted_pair"])
+
+
+@pytest.mark.parametrize("T,K,E,NS", [(14564, 8, 256, 1), (14563, 8, 255, 1), (30000, 10, 512, 1),
+                                      (114, 8, 256, 1), (113, 9, 9, 0)])
+def test_segmentation_block_round_edges(T, K, E, NS):
+    """One and several rounds per block (131072 pairs is the step), a last
+    block of few pairs, and the smallest multi-block batches."""
+    ids, wts = random_routing(T, K, E, seed=T, invalid_frac=0.02, zero_frac=0.02)
+    seg = _gpu_segment(ids, wts, E, NS, True)
+    ref = oracle.segment(ids, wts, E, NS, True)
+    np.testing.assert_array_equal(seg.seg_start.cpu().numpy(), ref["seg_start"])
+    for k in ("sorted_pair", "sorted_tok", "inv"):
+        np.testing.assert_array_equal(getattr(seg, k).cpu().numpy()[: seg.A], ref[k])
+
+
 @pytest.mark.parametrize("T,E,K,renorm", [(128, 8, 2, True), (500, 8, 2, True),
                                            (40, 32, 8, True), (300, 16, 3, False),
                                            (7, 8, 2, False)])

@@ -9,12 +9,14 @@
 // are formed by one thread in a fixed fp32 sequence (see xtu_expf).
 //
 // Segmentation: a stable counting sort of the flat (token, expert) pairs by
-// bucket, in three launches (per-block histogram in LDS, one-workgroup scan,
-// per-block stable scatter).  Ranks inside a block are exact: a wave finds
-// the lanes sharing its bucket with ballots, waves are ordered through LDS
-// counters, and blocks through the scanned histogram.
+// bucket, in two launches (per-block counts; every block sums all blocks'
+// counts and places its own pairs).  Ranks inside a block are exact: a wave
+// finds the lanes sharing its bucket with ballots, waves are ordered through
+// an LDS table of counts, and blocks through the summed counts.
 #include <mutex>
 #include <stdio.h>
+
+#include <type_traits>
 
 #include "route_tiny.hpp"
 #include "xtu_common.hpp"
@@ -294,16 +296,38 @@ void launch_route_wave(int epl, const float* logits, const float* bias, int T, i
 // ----------------------------------------------------------------------------
 // segmentation
 // ----------------------------------------------------------------------------
-constexpr int kSegThreads = 256;
-constexpr int kSegRounds = 16;
-constexpr int kSegChunk = kSegThreads * kSegRounds;   // pairs per block
+// A workgroup ranks one pair per thread and round: a wave finds the lanes
+// sharing its bucket with one ballot per bit of the bucket id and writes its
+// per-bucket counts as one row of a 16-bit [wave][bucket] table in LDS; an
+// exclusive prefix down the table's columns (two buckets per thread) orders
+// the waves.  A pair's position is then bucket start + its wave's prefix +
+// its rank in the wave: a fixed number of barriers per 1024 pairs, whatever
+// the bucket count.
+constexpr int kSegThreads = 1024;
+constexpr int kSegWaves = kSegThreads / kWave;
+// Blocks of a large batch: enough to spread the ranking over the chip, few
+// enough that every block can sum all blocks' counts by itself (128 blocks x
+// 514 buckets = 0.26 MB of L2 reads per block), which saves a scan launch.
+constexpr int kSegMaxBlocks = 128;
+// pairs per block of the workspace bound's first term (see
+// xtu_segment_workspace_bytes)
+constexpr int kSegBoundChunk = 4096;
 
 struct SegArgs {
   const int32_t* ids;
   const float* wts;
   const int32_t* id_map;   // optional id translation applied before bucketing
   int T, K, E, NS, drop_zero, A, NB;
+  int rounds;              // rounds of kSegThreads pairs per block
 };
+
+struct SegOut {
+  int32_t *seg_start, *active, *n_active, *tile_expert, *tile_row0, *n_tiles, *expert_tile_start;
+  int NB, bm, A;
+};
+
+// Buckets rounded up so that a table row is whole 16-byte pieces.
+__host__ __device__ constexpr int seg_nbp(int NB) { return (NB + 7) & ~7; }
 
 __device__ __forceinline__ int bucket_of(const SegArgs& a, int p, float* w_out, int* tok_out) {
   const int TK = a.T * a.K;
@@ -323,209 +347,6 @@ __device__ __forceinline__ int bucket_of(const SegArgs& a, int p, float* w_out, 
   return a.E + q % a.NS;
 }
 
-__global__ __launch_bounds__(kSegThreads) void seg_hist_kernel(SegArgs a,
-                                                               int32_t* __restrict__ bcnt) {
-  extern __shared__ int cnt[];
-  for (int e = threadIdx.x; e < a.NB; e += kSegThreads) cnt[e] = 0;
-  __syncthreads();
-  const int base = blockIdx.x * kSegChunk;
-  const int nrounds = min(kSegRounds, (a.A - base + kSegThreads - 1) / kSegThreads);
-  for (int r = 0; r < nrounds; ++r) {
-    const int p = base + r * kSegThreads + threadIdx.x;
-    if (p < a.A) {
-      float w;
-      int tok;
-      atomicAdd(&cnt[bucket_of(a, p, &w, &tok)], 1);
-    }
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < a.NB; e += kSegThreads)
-    bcnt[(size_t)blockIdx.x * a.NB + e] = cnt[e];
-}
-
-// One workgroup: per-bucket exclusive prefix over blocks (in place), bucket
-// totals, seg_start, the list of non-empty expert buckets and the GEMM tile
-// list (tiles of bm rows inside each non-trash bucket).
-__global__ __launch_bounds__(1024) void seg_scan_kernel(int NB, int nblocks, int bm,
-                                                        int32_t* __restrict__ bcnt,
-                                                        int32_t* __restrict__ seg_start,
-                                                        int32_t* __restrict__ active,
-                                                        int32_t* __restrict__ n_active,
-                                                        int32_t* __restrict__ tile_expert,
-                                                        int32_t* __restrict__ tile_row0,
-                                                        int32_t* __restrict__ n_tiles,
-                                                        int32_t* __restrict__ expert_tile_start) {
-  __shared__ int s_tot[2048];
-  __shared__ int s_act[2048];
-  __shared__ int s_til[2048];
-  __shared__ int s_part[3][32];
-  const int tid = threadIdx.x;
-  // per-bucket running sum over blocks
-  for (int e = tid; e < NB; e += 1024) {
-    int run = 0;
-    int b = 0;
-    for (; b + 4 <= nblocks; b += 4) {
-      const int c0 = bcnt[(size_t)(b + 0) * NB + e];
-      const int c1 = bcnt[(size_t)(b + 1) * NB + e];
-      const int c2 = bcnt[(size_t)(b + 2) * NB + e];
-      const int c3 = bcnt[(size_t)(b + 3) * NB + e];
-      bcnt[(size_t)(b + 0) * NB + e] = run;
-      bcnt[(size_t)(b + 1) * NB + e] = run + c0;
-      bcnt[(size_t)(b + 2) * NB + e] = run + c0 + c1;
-      bcnt[(size_t)(b + 3) * NB + e] = run + c0 + c1 + c2;
-      run += c0 + c1 + c2 + c3;
-    }
-    for (; b < nblocks; ++b) {
-      const int c = bcnt[(size_t)b * NB + e];
-      bcnt[(size_t)b * NB + e] = run;
-      run += c;
-    }
-    s_tot[e] = run;
-    const bool expert = e < NB - 1;   // last bucket is the trash bucket
-    s_act[e] = (expert && run > 0) ? 1 : 0;
-    s_til[e] = expert ? (run + bm - 1) / bm : 0;
-  }
-  __syncthreads();
-  // exclusive scans of s_tot, s_act, s_til over NB <= 2048 entries: each
-  // thread owns two consecutive entries; wave scans, then a scan of wave sums.
-  int v[3][2];
-  const int i0 = 2 * tid, i1 = 2 * tid + 1;
-  int* arr[3] = {s_tot, s_act, s_til};
-#pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    v[q][0] = i0 < NB ? arr[q][i0] : 0;
-    v[q][1] = i1 < NB ? arr[q][i1] : 0;
-  }
-  int incl[3];
-#pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    int s = v[q][0] + v[q][1];
-    const int lane = tid % 64;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int o = __shfl_up(s, off, 64);
-      if (lane >= off) s += o;
-    }
-    incl[q] = s;
-    if (lane == 63) s_part[q][tid / 64] = s;
-  }
-  __syncthreads();
-  if (tid < 32) {
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      int s = tid < 16 ? s_part[q][tid] : 0;
-      for (int off = 1; off < 32; off <<= 1) {
-        const int o = __shfl_up(s, off, 32);
-        if (tid >= off) s += o;
-      }
-      s_part[q][tid] = s;   // inclusive over waves
-    }
-  }
-  __syncthreads();
-  int ex[3][2];
-#pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    const int w = tid / 64;
-    const int wave_base = w > 0 ? s_part[q][w - 1] : 0;
-    const int excl = wave_base + incl[q] - (v[q][0] + v[q][1]);
-    ex[q][0] = excl;
-    ex[q][1] = excl + v[q][0];
-  }
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int e = 2 * tid + h;
-    if (e < NB) {
-      seg_start[e] = ex[0][h];
-      if (e == NB - 1) seg_start[NB] = ex[0][h] + v[0][h];
-      if (v[1][h]) active[ex[1][h]] = e;
-      expert_tile_start[e] = ex[2][h];
-      if (e == NB - 1) expert_tile_start[NB] = ex[2][h] + v[2][h];
-      const int nt = v[2][h];
-      for (int j = 0; j < nt; ++j) {
-        tile_expert[ex[2][h] + j] = e;
-        tile_row0[ex[2][h] + j] = ex[0][h] + j * bm;
-      }
-    }
-  }
-  if (tid == 1023) {
-    n_active[0] = s_part[1][15];
-    n_tiles[0] = s_part[2][15];
-  }
-}
-
-__global__ __launch_bounds__(kSegThreads) void seg_scatter_kernel(
-    SegArgs a, const int32_t* __restrict__ bexcl, const int32_t* __restrict__ seg_start,
-    int32_t* __restrict__ sorted_pair, int32_t* __restrict__ sorted_tok,
-    float* __restrict__ sorted_wts, int32_t* __restrict__ inv) {
-  extern __shared__ int lds[];
-  int* run = lds;                       // [NB] running count of this block
-  int* wcnt = lds + a.NB;               // [4][NB] per-wave counts of the round
-  const int wv = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  for (int e = threadIdx.x; e < a.NB; e += kSegThreads) {
-    run[e] = seg_start[e] + bexcl[(size_t)blockIdx.x * a.NB + e];
-    wcnt[e] = wcnt[a.NB + e] = wcnt[2 * a.NB + e] = wcnt[3 * a.NB + e] = 0;
-  }
-  __syncthreads();
-  const int base = blockIdx.x * kSegChunk;
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const int nbits = 32 - __builtin_clz(a.NB - 1);   // bits of the largest bucket id (NB >= 2)
-  // rounds holding pairs only (uniform: a short batch skips the empty ones)
-  const int nrounds = min(kSegRounds, (a.A - base + kSegThreads - 1) / kSegThreads);
-  for (int r = 0; r < nrounds; ++r) {
-    const int p = base + r * kSegThreads + threadIdx.x;
-    const bool valid = p < a.A;
-    float w = 0.f;
-    int tok = 0;
-    const int bk = valid ? bucket_of(a, p, &w, &tok) : -1;
-    // lanes of this wave that share my bucket: the valid lanes that agree
-    // with mine on every bit of the bucket id (one ballot per bit)
-    uint64_t m = __ballot(valid);
-    for (int bit = 0; bit < nbits; ++bit) {
-      const bool on = (bk >> bit) & 1;
-      const uint64_t b1 = __ballot(valid && on);
-      m &= on ? b1 : ~b1;
-    }
-    const int rank = __builtin_popcountll(m & lt_mask);
-    const int wcount = __builtin_popcountll(m);
-    const bool leader = valid && lane == __builtin_ctzll(m);
-    if (leader) wcnt[wv * a.NB + bk] = wcount;
-    __syncthreads();
-    if (valid) {
-      int before = 0;
-      for (int q = 0; q < wv; ++q) before += wcnt[q * a.NB + bk];
-      const int pos = run[bk] + before + rank;
-      sorted_pair[pos] = p;
-      sorted_tok[pos] = tok;
-      sorted_wts[pos] = w;
-      inv[p] = pos;
-    }
-    __syncthreads();
-    // advance the running counters and clear the round's wave counts
-    if (leader) {
-      // the last wave holding this bucket adds the whole round's count
-      int total = 0;
-      bool last = true;
-      for (int q = 0; q < 4; ++q) {
-        const int c = wcnt[q * a.NB + bk];
-        total += c;
-        if (q > wv && c > 0) last = false;
-      }
-      if (last) run[bk] += total;
-    }
-    __syncthreads();
-    if (leader) wcnt[wv * a.NB + bk] = 0;
-    __syncthreads();
-  }
-}
-
-// ----------------------------------------------------------------------------
-// Small batches (decode): routing and the whole segmentation in one
-// workgroup.  A = T*K + T*NS <= 1024 pairs, NB <= 2048 buckets.  Same
-// outputs, same order and same fp32 sequence as the multi-launch path.
-// ----------------------------------------------------------------------------
-constexpr int kSmallMaxA = 1024;
-constexpr int kSmallMaxNB = 2048;
-
 // Inclusive prefix sum across the 64 lanes of a wave (DPP row shifts, then
 // row broadcasts); lanes whose source is out of range add 0.
 __device__ __forceinline__ int wave_incl_scan(int x) {
@@ -538,42 +359,240 @@ __device__ __forceinline__ int wave_incl_scan(int x) {
   return x;
 }
 
+// Rank of this lane among the wave's valid lanes with its bucket b (below
+// 1 << nbits); `same` = those lanes.
+__device__ __forceinline__ int wave_bucket_rank(int b, bool valid, int nbits,
+                                                unsigned long long& same) {
+  unsigned long long m = __ballot(valid);
+  for (int bit = 0; bit < nbits; ++bit) {
+    const bool on = (b >> bit) & 1;
+    const unsigned long long b1 = __ballot(valid && on);
+    m &= on ? b1 : ~b1;
+  }
+  same = m;
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                   __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+__device__ __forceinline__ void clear_counts(uint16_t* wc, int nbp, int nw) {
+  for (int i = threadIdx.x; i < nw * nbp / 8; i += blockDim.x)
+    reinterpret_cast<u32x4_t*>(wc)[i] = u32x4_t{0u, 0u, 0u, 0u};
+}
+
+// Buckets 2t and 2t + 1 of thread t: the nw waves' counts become exclusive
+// prefixes in place; c0, c1 = the totals (at most 1024: 16-bit halves).
+__device__ __forceinline__ void column_prefix(uint16_t* wc, int nbp, int nw, int t, int& c0,
+                                              int& c1) {
+  uint32_t* col = reinterpret_cast<uint32_t*>(wc) + t;
+  uint32_t c[kSegWaves], run = 0u;
+#pragma unroll
+  for (int w = 0; w < kSegWaves; ++w) c[w] = w < nw ? col[w * (nbp / 2)] : 0u;
+#pragma unroll
+  for (int w = 0; w < kSegWaves; ++w) {
+    if (w < nw) col[w * (nbp / 2)] = run;
+    run += c[w];
+  }
+  c0 = (int)(run & 0xffffu);
+  c1 = (int)(run >> 16);
+}
+
+// Bucket totals c0, c1 of thread t's buckets (2t, 2t + 1) -> their first
+// rows; with `write`, seg_start, the list of non-empty expert buckets and the
+// GEMM tile list (tiles of bm rows inside each non-trash bucket).  Called by
+// the whole block (kSegThreads or fewer threads, at least NB / 2).
+__device__ __forceinline__ void bucket_starts(const SegOut& o, int t, int c0, int c1, bool write,
+                                              int (*wsum)[kSegWaves], int& s0, int& s1) {
+  const int NB = o.NB, e0 = 2 * t;
+  // the last bucket is the trash bucket
+  const bool x0 = e0 < NB - 1, x1 = e0 + 1 < NB - 1;
+  const int n0 = x0 ? (c0 + o.bm - 1) / o.bm : 0, n1 = x1 ? (c1 + o.bm - 1) / o.bm : 0;
+  const int a0 = x0 && c0 > 0 ? 1 : 0, a1 = x1 && c1 > 0 ? 1 : 0;
+  const int lane = t % kWave, wv = t / kWave, nwv = (int)blockDim.x / kWave;
+  const int ir = wave_incl_scan(c0 + c1), ia = wave_incl_scan(a0 + a1),
+            it = wave_incl_scan(n0 + n1);
+  if (lane == kWave - 1) {
+    wsum[0][wv] = ir;
+    wsum[1][wv] = ia;
+    wsum[2][wv] = it;
+  }
+  __syncthreads();
+  int br = ir - c0 - c1, ba = ia - a0 - a1, bt = it - n0 - n1, na = 0, nt = 0;
+#pragma unroll
+  for (int q = 0; q < kSegWaves; ++q) {
+    if (q < nwv) {
+      const int r = wsum[0][q], c = wsum[1][q], n = wsum[2][q];
+      if (q < wv) {
+        br += r;
+        ba += c;
+        bt += n;
+      }
+      na += c;
+      nt += n;
+    }
+  }
+  s0 = br;
+  s1 = br + c0;
+  if (!write) return;
+  if (e0 < NB) {
+    o.seg_start[e0] = s0;
+    o.expert_tile_start[e0] = bt;
+  }
+  if (e0 + 1 < NB) {
+    o.seg_start[e0 + 1] = s1;
+    o.expert_tile_start[e0 + 1] = bt + n0;
+  }
+  if (a0) o.active[ba] = e0;
+  if (a1) o.active[ba + a0] = e0 + 1;
+  for (int j = 0; j < n0; ++j) {
+    o.tile_expert[bt + j] = e0;
+    o.tile_row0[bt + j] = s0 + j * o.bm;
+  }
+  for (int j = 0; j < n1; ++j) {
+    o.tile_expert[bt + n0 + j] = e0 + 1;
+    o.tile_row0[bt + n0 + j] = s1 + j * o.bm;
+  }
+  if (t == 0) {
+    o.seg_start[NB] = o.A;
+    o.expert_tile_start[NB] = nt;
+    o.n_active[0] = na;
+    o.n_tiles[0] = nt;
+  }
+}
+
+// Bucket counts of each block's pairs: bcnt[block][nbp].
+__global__ __launch_bounds__(kSegThreads) void seg_count_kernel(SegArgs a,
+                                                                int32_t* __restrict__ bcnt) {
+  extern __shared__ int cnt[];
+  const int nbp = seg_nbp(a.NB);
+  for (int e = threadIdx.x; e < nbp; e += kSegThreads) cnt[e] = 0;
+  __syncthreads();
+  const int base = blockIdx.x * a.rounds * kSegThreads;
+  for (int r = 0; r < a.rounds; ++r) {
+    const int p = base + r * kSegThreads + threadIdx.x;
+    if (p < a.A) {
+      float w;
+      int tok;
+      atomicAdd(&cnt[bucket_of(a, p, &w, &tok)], 1);
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < nbp; e += kSegThreads)
+    bcnt[(size_t)blockIdx.x * nbp + e] = cnt[e];
+}
+
+// Every block sums all blocks' counts for itself (bucket totals and the part
+// before this block; nblocks <= kSegMaxBlocks), scans the totals and places
+// its own pairs; block 0 also writes the bucket starts and tile lists.
+// Latency bound.
+__global__ __launch_bounds__(kSegThreads) void seg_place_kernel(
+    SegArgs a, SegOut o, const int32_t* __restrict__ bcnt, int nblocks,
+    int32_t* __restrict__ sorted_pair, int32_t* __restrict__ sorted_tok,
+    float* __restrict__ sorted_wts, int32_t* __restrict__ inv) {
+  extern __shared__ __attribute__((aligned(16))) int place_lds[];
+  __shared__ int wsum[3][kSegWaves];
+  const int nbp = seg_nbp(a.NB), half = nbp / 2;
+  int* base = place_lds;   // [nbp] pairs of earlier blocks, then this block's next rows
+  uint16_t* wc = reinterpret_cast<uint16_t*>(place_lds + nbp);   // [waves][nbp]
+  int* tot = place_lds + nbp;   // [nbp] bucket totals, before wc is used
+  const int tid = threadIdx.x, wv = tid / kWave;
+  const int p0 = blockIdx.x * a.rounds * kSegThreads;
+  // this thread's first pair, in flight beside the counts
+  float w = 0.f;
+  int tok = 0;
+  int b = p0 + tid < a.A ? bucket_of(a, p0 + tid, &w, &tok) : -1;
+  for (int e = tid; e < 2 * nbp; e += kSegThreads) place_lds[e] = 0;
+  __syncthreads();
+  // thread groups of gs threads each take every ng-th block's counts
+  const int gs = (half + kWave - 1) / kWave * kWave, ng = kSegThreads / gs;
+  const int g = tid / gs, t = tid % gs;
+  if (g < ng && t < half) {
+    int t0 = 0, t1 = 0, b0 = 0, b1 = 0;
+#pragma unroll 8
+    for (int j = g; j < nblocks; j += ng) {
+      const int2 c = reinterpret_cast<const int2*>(bcnt + (size_t)j * nbp)[t];
+      t0 += c.x;
+      t1 += c.y;
+      if (j < (int)blockIdx.x) {
+        b0 += c.x;
+        b1 += c.y;
+      }
+    }
+    atomicAdd(&tot[2 * t], t0);
+    atomicAdd(&tot[2 * t + 1], t1);
+    atomicAdd(&base[2 * t], b0);
+    atomicAdd(&base[2 * t + 1], b1);
+  }
+  __syncthreads();
+  int s0, s1;
+  {
+    const int c0 = tid < half ? tot[2 * tid] : 0, c1 = tid < half ? tot[2 * tid + 1] : 0;
+    bucket_starts(o, tid, c0, c1, blockIdx.x == 0, wsum, s0, s1);   // one barrier inside
+  }
+  if (tid < half) {
+    base[2 * tid] += s0;
+    base[2 * tid + 1] += s1;
+  }
+  const int nbits = 32 - __builtin_clz(a.NB - 1);   // bits of the largest bucket id (NB >= 2)
+  for (int r = 0; r < a.rounds; ++r) {
+    const int p = p0 + r * kSegThreads + tid;
+    if (p - tid >= a.A) break;   // whole block
+    if (r > 0) b = p < a.A ? bucket_of(a, p, &w, &tok) : -1;
+    const bool valid = b >= 0;
+    unsigned long long same;
+    const int rank = wave_bucket_rank(b, valid, nbits, same);
+    clear_counts(wc, nbp, kSegWaves);
+    __syncthreads();
+    if (valid && rank == 0) wc[wv * nbp + b] = (uint16_t)__popcll(same);
+    __syncthreads();
+    int c0 = 0, c1 = 0;
+    if (tid < half) column_prefix(wc, nbp, kSegWaves, tid, c0, c1);
+    __syncthreads();
+    if (valid) {
+      const int pos = base[b] + wc[wv * nbp + b] + rank;
+      sorted_pair[pos] = p;
+      sorted_tok[pos] = tok;
+      sorted_wts[pos] = w;
+      inv[p] = pos;
+    }
+    if (r + 1 < a.rounds) {
+      __syncthreads();
+      if (tid < half) {
+        base[2 * tid] += c0;
+        base[2 * tid + 1] += c1;
+      }
+    }
+  }
+}
+
+// ----------------------------------------------------------------------------
+// Small batches (decode): routing and the whole segmentation in one
+// workgroup.  A = T*K + T*NS <= 1024 pairs, NB <= 2048 buckets.  Same
+// outputs, same order and same fp32 sequence as the multi-launch path.
+// ----------------------------------------------------------------------------
+constexpr int kSmallMaxA = 1024;
+constexpr int kSmallMaxNB = 2048;
+static_assert(kSmallMaxA <= kSegThreads && kSmallMaxNB <= 2 * kSegThreads,
+              "one pair and two buckets per thread");
+
 constexpr int kFewNB = 64;   // bucket count of the ballot segmentation
 
-struct SegSmem {
-  int ids[kSmallMaxA];
-  float w[kSmallMaxA];
-  int bk[kSmallMaxA];
-  int cnt[kSmallMaxNB];
-  int wsum[3][16];
-  int wc[kFewNB][16];          // ballot segmentation: pairs of bucket v in wave q
+struct FewSmem {
+  int wc[kFewNB][kSegWaves];   // pairs of bucket v in wave q
   int bstart[kFewNB];
 };
 
-// Stable counting sort of the A <= NT pairs (pair p in thread p) over NB <=
-// kFewNB buckets: per wave, one ballot per bucket gives each pair its rank
+// Few buckets: a stable counting sort of the A pairs (pair p in thread p) over
+// NB <= kFewNB buckets.  Per wave, one ballot per bucket gives each pair its rank
 // among the wave's pairs of its bucket and the wave's count; one wave scans
 // the bucket totals.  Position = bucket start + the bucket's pairs in
-// earlier waves + rank: the same stable order as the counting sort.
-template <int NT>
-__device__ __forceinline__ void segment_few_buckets(const SmallArgs& a, SegSmem& g, int A, int TK,
-                                                    int NB) {
-  constexpr int NW = NT / kWave;
+// earlier waves + rank: the same stable order.  Two barriers fewer than the
+// count table: tiny Mixtral's layer (256 pairs over 9 buckets) 40.5 us against
+// 41.1.
+__device__ __forceinline__ void segment_few_buckets(const SmallArgs& a, FewSmem& g, int b, float w,
+                                                    int A, int TK, int NB) {
+  const int NW = blockDim.x / kWave;
   const int tid = threadIdx.x, lane = tid % kWave, wv = tid / kWave;
-  const int K = a.K, E = a.E, NS = a.NS;
-  int b = -1;
-  float w = 1.0f;
-  if (tid < A) {
-    if (tid < TK) {
-      int e = g.ids[tid];
-      w = g.w[tid];
-      if (a.id_map && e >= 0 && e < E) e = a.id_map[e];
-      b = (e < 0 || e >= E) ? (E + NS) : e;
-      if (a.drop_zero && w == 0.0f) b = E + NS;
-    } else {
-      b = E + (tid - TK) % NS;
-    }
-  }
+  const int K = a.K, NS = a.NS;
   int rank = 0;
   for (int v = 0; v < NB; ++v) {
     const unsigned long long m = __ballot(b == v);
@@ -623,7 +642,7 @@ __device__ __forceinline__ void segment_few_buckets(const SmallArgs& a, SegSmem&
     a.sorted_pair[pos] = tid;
     a.inv[tid] = pos;
     a.sorted_tok[pos] = tid < TK ? tid / K : (tid - TK) / NS;
-    a.sorted_wts[pos] = tid < TK ? w : 1.0f;
+    a.sorted_wts[pos] = w;
   }
 }
 
@@ -688,148 +707,100 @@ __device__ __forceinline__ void route_token_lane(const float* __restrict__ l, in
   }
 }
 
-// One workgroup of NT threads.  MODE 0: softmax routing, 1: grouped sigmoid
-// routing (NT/256 teams route that many tokens at a time; LANE: softmax over
-// at most kLaneE experts, one thread per token), 2: ids/wts given.  Then the
-// whole segmentation.
-template <int MODE, int NT, bool LANE = false, bool FEW = false>
-__global__ __launch_bounds__(NT) void route_seg_small_kernel(SmallArgs a) {
-  __shared__ SegSmem g;
-  extern __shared__ float route_lds[];
-  constexpr int NW = NT / kWave;
-  const int tid = threadIdx.x;
+// How route_seg_small_kernel routes its tokens: 256-thread teams, softmax by
+// one thread per token (at most kLaneE experts), or one wave per token with
+// 4 / 8 experts per lane (E = 256 / 512).
+enum SmallRoute : int { kTeams = 0, kLanes = 1, kWave4 = 4, kWave8 = 8 };
+
+// One workgroup of at least A threads and NB / 2 threads.  MODE 0: softmax
+// routing, 1: grouped sigmoid routing, 2: ids/wts given.  Then the whole
+// segmentation, one pair per thread (FEW: over at most kFewNB buckets).  Latency bound (one workgroup): with
+// the pairs ranked by ballots instead of each pair scanning the pairs before
+// it, 1023 pairs over 514 buckets 36.0 -> 6.0 us; with one wave per token
+// instead of four 256-thread teams in lockstep, T = 16 grouped sigmoid over
+// 256 experts 35.5 -> 8.8 us (routing and segmentation).
+template <int MODE, int RT, bool FEW>
+__global__ __launch_bounds__(kSegThreads) void route_seg_small_kernel(SmallArgs a) {
+  __shared__ int s_ids[kSmallMaxA];
+  __shared__ float s_w[kSmallMaxA];
+  __shared__ int s_start[kSmallMaxNB];
+  __shared__ int wsum[3][kSegWaves];
+  extern __shared__ __attribute__((aligned(16))) float small_lds[];
+  const int tid = threadIdx.x, wv = tid / kWave;
   const int T = a.T, K = a.K, E = a.E, NS = a.NS;
-  const int TK = T * K, A = TK + T * NS, NB = E + NS + 1;
-  if (MODE == 0 && LANE) {
-    for (int t = tid; t < T; t += NT)
-      route_token_lane(a.logits + (long)t * E, E, K, a.renorm, a.ids + (long)t * K,
-                       a.wts + (long)t * K, g.ids + t * K, g.w + t * K);
-  } else if (MODE < 2) {
-    // NT / 256 teams of 256 threads route that many tokens at a time
-    constexpr int NTEAM = NT / 256;
-    const int team = tid / 256, ttid = tid % 256;
-    const int nc = (MODE == 1 ? a.n_group : (E + 31) / 32) * K;
-    const RouteScratch s(route_lds + team * route_team_words(E, nc), E, nc);
-    for (int t0 = 0; t0 < T; t0 += NTEAM) {
-      const int t = t0 + team;
-      const bool valid = t < T;
-      route_token<MODE < 2 ? MODE : 0, 256>(a.logits + (long)t * E, a.bias, E, K, a.n_group,
-                                             a.topk_group, a.scale, a.renorm, s, ttid, valid,
-                                             a.ids + (long)t * K, a.wts + (long)t * K,
-                                             g.ids + t * K, g.w + t * K);
+  const int TK = T * K, A = TK + T * NS, NB = E + NS + 1, trash = E + NS;
+  if constexpr (MODE < 2) {
+    if constexpr (RT == kLanes) {
+      for (int t = tid; t < T; t += blockDim.x)
+        route_token_lane(a.logits + (long)t * E, E, K, a.renorm, a.ids + (long)t * K,
+                         a.wts + (long)t * K, s_ids + t * K, s_w + t * K);
+    } else if constexpr (RT == kTeams) {
+      // blockDim / 256 teams of 256 threads route that many tokens at a time
+      const int nteam = blockDim.x / 256, team = tid / 256, ttid = tid % 256;
+      const int nc = (MODE == 1 ? a.n_group : (E + 31) / 32) * K;
+      const RouteScratch s(small_lds + team * route_team_words(E, nc), E, nc);
+      for (int t0 = 0; t0 < T; t0 += nteam) {
+        const int t = t0 + team;
+        const bool valid = t < T;
+        route_token<MODE, 256>(a.logits + (long)t * E, a.bias, E, K, a.n_group, a.topk_group,
+                               a.scale, a.renorm, s, ttid, valid, a.ids + (long)t * K,
+                               a.wts + (long)t * K, s_ids + t * K, s_w + t * K);
+      }
+    } else {
+      const int nw = blockDim.x / kWave;
+      for (int t = wv; t < T; t += nw)
+        tiny::route_token_wave<MODE, RT>(a.logits + (long)t * E, a.bias, K, a.n_group,
+                                         a.topk_group, a.scale, a.renorm, tid % kWave,
+                                         a.ids + (long)t * K, a.wts + (long)t * K,
+                                         s_ids + t * K, s_w + t * K);
     }
-  } else {
-    for (int p = tid; p < TK; p += NT) {
-      g.ids[p] = a.ids[p];
-      g.w[p] = a.wts[p];
-    }
+    __syncthreads();   // the routing's scratch becomes the count table
   }
-  if constexpr (FEW) {   // A <= NT pairs over NB <= kFewNB buckets
-    __syncthreads();
-    segment_few_buckets<NT>(a, g, A, TK, NB);
+  uint16_t* wc = reinterpret_cast<uint16_t*>(small_lds);   // [waves holding pairs][nbp]
+  const int nbp = seg_nbp(NB), half = nbp / 2, nw = (A + kWave - 1) / kWave;
+  int b = -1;
+  float w = 1.0f;
+  if (tid < TK) {
+    int e;
+    if constexpr (MODE < 2) {
+      e = s_ids[tid];
+      w = s_w[tid];
+    } else {
+      e = a.ids[tid];
+      w = a.wts[tid];
+    }
+    if (a.id_map && e >= 0 && e < E) e = a.id_map[e];
+    b = (e < 0 || e >= E) ? trash : e;
+    if (a.drop_zero && w == 0.0f) b = trash;
+  } else if (tid < A) {
+    b = E + (tid - TK) % NS;
+  }
+  if constexpr (FEW) {
+    __shared__ FewSmem few;
+    segment_few_buckets(a, few, b, w, A, TK, NB);
     return;
   }
-  for (int e = tid; e < NB; e += NT) g.cnt[e] = 0;
+  clear_counts(wc, nbp, nw);
+  const bool valid = b >= 0;
+  unsigned long long same;
+  const int rank = wave_bucket_rank(b, valid, 32 - __builtin_clz(NB - 1), same);
   __syncthreads();
-  for (int p = tid; p < A; p += NT) {
-    int b;
-    if (p < TK) {
-      int e = g.ids[p];
-      if (a.id_map && e >= 0 && e < E) e = a.id_map[e];
-      b = (e < 0 || e >= E) ? (E + NS) : e;
-      if (a.drop_zero && g.w[p] == 0.0f) b = E + NS;
-    } else {
-      b = E + (p - TK) % NS;
-    }
-    g.bk[p] = b;
-    atomicAdd(&g.cnt[b], 1);
-  }
-  for (int p = A + tid; p < ((A + 3) & ~3); p += NT) g.bk[p] = -1;   // pad for 4-wide reads
+  if (valid && rank == 0) wc[wv * nbp + b] = (uint16_t)__popcll(same);
   __syncthreads();
-  // one scan pass over the buckets for (rows, active flag, tiles): each thread
-  // owns `per` consecutive buckets
-  const int per = (NB + NT - 1) / NT;
-  const int lane = tid % kWave, wv = tid / kWave;
-  int c_loc[8], s_rows = 0, s_act = 0, s_til = 0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int e = tid * per + i;
-    const int c = (i < per && e < NB) ? g.cnt[e] : 0;
-    c_loc[i] = c;
-    s_rows += c;
-    s_act += (e < NB - 1 && c > 0) ? 1 : 0;
-    s_til += (e < NB - 1) ? (c + a.bm - 1) / a.bm : 0;
-  }
-  const int i_rows = wave_incl_scan(s_rows), i_act = wave_incl_scan(s_act),
-            i_til = wave_incl_scan(s_til);
-  if (lane == kWave - 1) {
-    g.wsum[0][wv] = i_rows;
-    g.wsum[1][wv] = i_act;
-    g.wsum[2][wv] = i_til;
-  }
+  int c0 = 0, c1 = 0, s0, s1;
+  if (tid < half) column_prefix(wc, nbp, nw, tid, c0, c1);
+  const SegOut o{a.seg_start, a.active, a.n_active, a.tile_expert, a.tile_row0, a.n_tiles,
+                 a.expert_tile_start, NB, a.bm, A};
+  bucket_starts(o, tid, c0, c1, true, wsum, s0, s1);
+  if (2 * tid < NB) s_start[2 * tid] = s0;
+  if (2 * tid + 1 < NB) s_start[2 * tid + 1] = s1;
   __syncthreads();
-  int b_rows = i_rows - s_rows, b_act = i_act - s_act, b_til = i_til - s_til;
-  int n_act = 0, n_til = 0;
-#pragma unroll
-  for (int q = 0; q < NW; ++q) {
-    if (q < wv) {
-      b_rows += g.wsum[0][q];
-      b_act += g.wsum[1][q];
-      b_til += g.wsum[2][q];
-    }
-    n_act += g.wsum[1][q];
-    n_til += g.wsum[2][q];
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int e = tid * per + i;
-    if (i < per && e < NB) {
-      const int c = c_loc[i];
-      a.seg_start[e] = b_rows;
-      a.expert_tile_start[e] = b_til;
-      g.cnt[e] = b_rows;   // bucket start, for the scatter below
-      if (e < NB - 1 && c > 0) {
-        a.active[b_act++] = e;
-        const int nt = (c + a.bm - 1) / a.bm;
-        for (int j = 0; j < nt; ++j) {
-          a.tile_expert[b_til + j] = e;
-          a.tile_row0[b_til + j] = b_rows + j * a.bm;
-        }
-        b_til += nt;
-      }
-      b_rows += c;
-      if (e == NB - 1) {
-        a.seg_start[NB] = A;
-        a.expert_tile_start[NB] = n_til;
-      }
-    }
-  }
-  if (tid == 0) {
-    a.n_active[0] = n_act;
-    a.n_tiles[0] = n_til;
-  }
-  __syncthreads();
-  // stable scatter: position = bucket start + earlier pairs of the bucket
-  for (int p = tid; p < A; p += NT) {
-    const int b = g.bk[p];
-    int r = 0;
-    int q = 0;
-#pragma unroll 4
-    for (; q + 4 <= p; q += 4) {
-      const i32x4_t v = *reinterpret_cast<const i32x4_t*>(g.bk + q);
-      r += (v[0] == b) + (v[1] == b) + (v[2] == b) + (v[3] == b);
-    }
-    for (; q < p; ++q) r += g.bk[q] == b;
-    const int pos = g.cnt[b] + r;
-    a.sorted_pair[pos] = p;
-    a.inv[p] = pos;
-    if (p < TK) {
-      a.sorted_tok[pos] = p / K;
-      a.sorted_wts[pos] = g.w[p];
-    } else {
-      a.sorted_tok[pos] = (p - TK) / NS;
-      a.sorted_wts[pos] = 1.0f;
-    }
+  if (valid) {
+    const int pos = s_start[b] + wc[wv * nbp + b] + rank;
+    a.sorted_pair[pos] = tid;
+    a.inv[tid] = pos;
+    a.sorted_tok[pos] = tid < TK ? tid / K : (tid - TK) / NS;
+    a.sorted_wts[pos] = w;
   }
 }
 
@@ -858,25 +829,44 @@ hipError_t launch_small(const SmallArgs& a, hipStream_t stream) {
     }
     return hipSuccess;
   }
-  // few buckets: the ballot segmentation, one pair per thread
-  const long A = (long)a.T * a.K + (long)a.T * a.NS;
-  const bool few = a.E + a.NS + 1 <= kFewNB && A <= 1024;
+  const int A = a.T * a.K + a.T * a.NS, nbp = seg_nbp(a.E + a.NS + 1);
+  // threads of the segmentation: one pair and two buckets each
+  int threads = A > nbp / 2 ? A : nbp / 2;
+  const size_t table = (size_t)((A + kWave - 1) / kWave) * nbp * sizeof(uint16_t);
+  auto launch = [&](auto rt_tag, int route_threads, size_t route_lds) {
+    if (threads < route_threads) threads = route_threads;
+    threads = (threads + kWave - 1) / kWave * kWave;
+    // team routing: whole teams only
+    if (decltype(rt_tag)::value == kTeams && MODE < 2) threads = (threads + 255) / 256 * 256;
+    const size_t teams = decltype(rt_tag)::value == kTeams && MODE < 2 ? threads / 256 : 1;
+    const size_t lds = teams * route_lds > table ? teams * route_lds : table;
+    constexpr int RT = decltype(rt_tag)::value;
+    if constexpr (RT < kWave4) {   // the wave routers' E is past kFewNB
+      if (a.E + a.NS + 1 <= kFewNB) {
+        route_seg_small_kernel<MODE, RT, true><<<1, threads, lds, stream>>>(a);
+        return;
+      }
+    }
+    route_seg_small_kernel<MODE, RT, false><<<1, threads, lds, stream>>>(a);
+  };
+  using Lanes = std::integral_constant<int, kLanes>;
+  using Teams = std::integral_constant<int, kTeams>;
   if constexpr (MODE == 2) {
-    if (few && A <= 256) route_seg_small_kernel<2, 256, false, true><<<1, 256, 0, stream>>>(a);
-    else if (few) route_seg_small_kernel<2, 1024, false, true><<<1, 1024, 0, stream>>>(a);
-    else route_seg_small_kernel<MODE, 256><<<1, 256, 0, stream>>>(a);
-  } else if (MODE == 0 && a.E <= kLaneE && a.K <= kLaneK && few) {
-    // few experts and few buckets (shared experts included): one thread per
-    // token, no routing barriers, the ballot segmentation
-    if (A <= 256) route_seg_small_kernel<0, 256, true, true><<<1, 256, 0, stream>>>(a);
-    else route_seg_small_kernel<0, 1024, true, true><<<1, 1024, 0, stream>>>(a);
+    launch(Teams{}, kWave, 0);
   } else {
-    const int nc = (MODE == 1 ? a.n_group : (a.E + 31) / 32) * a.K;
-    const size_t team_lds = route_team_words(a.E, nc) * sizeof(float);
-    if (a.T <= 2)   // one team: fewer waves in lockstep through the barriers
-      route_seg_small_kernel<MODE, 256><<<1, 256, team_lds, stream>>>(a);
-    else
-      route_seg_small_kernel<MODE, 1024><<<1, 1024, 4 * team_lds, stream>>>(a);
+    const int wepl = tiny::wave_epl(MODE, a.E, a.n_group, a.renorm, a.logits, a.bias);
+    if (MODE == 0 && a.E <= kLaneE && a.K <= kLaneK) {
+      // few experts: one thread per token, no routing barriers
+      launch(Lanes{}, kWave, 0);
+    } else if (wepl != 0) {
+      const int rt = kWave * (a.T < kSegWaves ? a.T : kSegWaves);
+      if (wepl == 4) launch(std::integral_constant<int, kWave4>{}, rt, 0);
+      else launch(std::integral_constant<int, kWave8>{}, rt, 0);
+    } else {
+      const int nc = (MODE == 1 ? a.n_group : (a.E + 31) / 32) * a.K;
+      // one team for at most two tokens: fewer waves in lockstep through the barriers
+      launch(Teams{}, a.T <= 2 ? 256 : 1024, route_team_words(a.E, nc) * sizeof(float));
+    }
   }
   return hipSuccess;
 }
@@ -925,11 +915,19 @@ hipError_t xtu_route_grouped_sigmoid(const float* logits, const float* bias, int
   return hipPeekAtLastError();
 }
 
+// The counts of the blocks (at most kSegMaxBlocks; the bound grows with T,
+// so a workspace sized for more tokens holds fewer), and never less than one
+// row of counts per kSegBoundChunk pairs: xtu_segment_noalloc refuses the
+// shapes whose bound passes its static scratch.
 size_t xtu_segment_workspace_bytes(int T, int K, int E, int n_shared) {
   const long A = (long)T * K + (long)T * n_shared;
   const long NB = E + n_shared + 1;
-  const long nblocks = (A + kSegChunk - 1) / kSegChunk;
-  return (size_t)((nblocks > 0 ? nblocks : 1) * NB * sizeof(int32_t));
+  const long bound = (A + kSegBoundChunk - 1) / kSegBoundChunk;
+  long nblocks = (A + kSegThreads - 1) / kSegThreads;
+  if (nblocks > kSegMaxBlocks) nblocks = kSegMaxBlocks;
+  const size_t b0 = (size_t)((bound > 0 ? bound : 1) * NB * sizeof(int32_t));
+  const size_t b1 = (size_t)((nblocks > 0 ? nblocks : 1) * seg_nbp((int)NB) * sizeof(int32_t));
+  return b0 > b1 ? b0 : b1;
 }
 
 int xtu_segment_max_tiles(int T, int K, int E, int n_shared, int bm) {
@@ -943,9 +941,13 @@ int xtu_segment_max_tiles(int T, int K, int E, int n_shared, int bm) {
 namespace xtu {
 namespace {
 
-// The three segmentation launches over a caller-supplied workspace of
-// xtu_segment_workspace_bytes() bytes (every word written by seg_hist_kernel
-// before seg_scan_kernel reads it, so it needs no clearing).
+// The two segmentation launches over a caller-supplied workspace of
+// xtu_segment_workspace_bytes() bytes (every word written by seg_count_kernel
+// before seg_place_kernel reads it, so it needs no clearing).  Latency bound:
+// 45k pairs over 514 buckets 15.7 us, 74k over 258 16.9 us, 1.9k 11.4 us
+// (4.7 of it the counts); a histogram, a one-block scan and a scatter of
+// 4096-pair blocks, 16 rounds of four barriers each, took 43.2, 46.6 and
+// 23.3 us.
 hipError_t segment_impl(const int32_t* topk_ids, const float* topk_weights,
                         const int32_t* id_map, int T, int K, int E, int n_shared, int drop_zero,
                         int bm, void* workspace, int32_t* sorted_pair, int32_t* sorted_tok,
@@ -961,19 +963,20 @@ hipError_t segment_impl(const int32_t* topk_ids, const float* topk_weights,
                 n_tiles && expert_tile_start);
   XTU_CHECK_ARG(A == 0 || (sorted_pair && sorted_tok && sorted_wts && inv));
   XTU_CHECK_ARG(T * K == 0 || (topk_ids && topk_weights));
-  const int nblocks = (int)((A + kSegChunk - 1) / kSegChunk);
-  SegArgs a{topk_ids, topk_weights, id_map, T, K, E, n_shared, drop_zero, (int)A, NB};
+  const int rounds = (int)((A + (long)kSegThreads * kSegMaxBlocks - 1) /
+                           ((long)kSegThreads * kSegMaxBlocks));
+  const long chunk = (long)(rounds > 0 ? rounds : 1) * kSegThreads;
+  const int nblocks = (int)((A + chunk - 1) / chunk);
+  const int nbp = seg_nbp(NB);
+  SegArgs a{topk_ids, topk_weights, id_map, T, K, E, n_shared, drop_zero, (int)A, NB, rounds};
+  SegOut o{seg_start, active, n_active, tile_expert, tile_row0, n_tiles, expert_tile_start, NB,
+           bm, (int)A};
   int32_t* bcnt = (int32_t*)workspace;
   (void)hipGetLastError();
-  if (nblocks > 0) {
-    seg_hist_kernel<<<nblocks, kSegThreads, NB * sizeof(int), stream>>>(a, bcnt);
-  }
-  seg_scan_kernel<<<1, 1024, 0, stream>>>(NB, nblocks, bm, bcnt, seg_start, active, n_active,
-                                          tile_expert, tile_row0, n_tiles, expert_tile_start);
-  if (nblocks > 0) {
-    seg_scatter_kernel<<<nblocks, kSegThreads, 5 * NB * sizeof(int), stream>>>(
-        a, bcnt, seg_start, sorted_pair, sorted_tok, sorted_wts, inv);
-  }
+  if (nblocks > 0) seg_count_kernel<<<nblocks, kSegThreads, nbp * sizeof(int), stream>>>(a, bcnt);
+  const size_t table = (size_t)kSegWaves * nbp * sizeof(uint16_t);   // >= the totals' nbp words
+  seg_place_kernel<<<nblocks > 0 ? nblocks : 1, kSegThreads, nbp * sizeof(int) + table, stream>>>(
+      a, o, bcnt, nblocks, sorted_pair, sorted_tok, sorted_wts, inv);
   return hipPeekAtLastError();
 }
 
