@@ -289,6 +289,32 @@ hipError_t xtu_decode_down_combine(int fmt, const void* act, const void* act_sha
                                    const int32_t* n_active, int max_active, void* out,
                                    int out_bf16, hipStream_t stream);
 
+/* ------------------------------------------- grouped GEMM, few rows per expert
+ * The same products as xtu_gemm_gate_up / xtu_gemm_down below (same layouts,
+ * same outputs; FP8 exact, its block scale applied to the fp32 sum of 128 k)
+ * for batches that are a weight stream: tiles of at most bm rows from the
+ * segmentation's tile list (bm <= xtu_stream_max_tile_m(fmt), the height it
+ * was built with), weights four super-blocks ahead in registers.  T: rows of
+ * x.  xtu_stream_down: sorted_pair non-null writes y rows in flat pair order
+ * (as xtu_decode_down_by_pair).  Requires H % 256 == 0, I % 128 == 0.
+ * xtu_decode_gate_up_fast: whether a decode batch of T rows takes the fast
+ * form of xtu_decode_gate_up (every row staged, one round per wave). */
+int xtu_stream_max_tile_m(int fmt);
+hipError_t xtu_stream_gate_up(int fmt, const void* x, int T, const int32_t* sorted_tok, int H,
+                              int I, const void* w13, const void* s13, const float* gs13,
+                              long w_estride, long s_estride, const int32_t* slot_map,
+                              const int32_t* seg_start, const int32_t* tile_expert,
+                              const int32_t* tile_row0, const int32_t* tile_lo,
+                              const int32_t* tile_hi, int bm, int max_tiles, void* act,
+                              float limit, float alpha, float beta, hipStream_t stream);
+hipError_t xtu_stream_down(int fmt, const void* act, int H, int I, const void* w2, const void* s2,
+                           const float* gs2, long w_estride, long s_estride,
+                           const int32_t* slot_map, const int32_t* seg_start,
+                           const int32_t* tile_expert, const int32_t* tile_row0,
+                           const int32_t* tile_lo, const int32_t* tile_hi, int bm, int max_tiles,
+                           const int32_t* sorted_pair, float* y, hipStream_t stream);
+int xtu_decode_gate_up_fast(int fmt, int T, int H);
+
 /* ------------------------------------------------ grouped GEMM (prefill) path
  * Replaces _gate_up_kernel / _down_kernel (vllm_xiaotu_moe/gpu_prefill.py:
  * 232-390) and gate_up_kernel_fp8 / down_kernel_fp8

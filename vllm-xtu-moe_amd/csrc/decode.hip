@@ -281,6 +281,11 @@ hipError_t xtu_decode_down_by_pair(int fmt, const void* act, int T, int H, int I
   return dispatch_decode(fmt, 1, a, max_active, stream);
 }
 
+int xtu_decode_gate_up_fast(int fmt, int T, int H) {
+  int ksplit = 0, xc = 0;
+  return H > 0 && H % 128 == 0 && gate_up_fast_shape_fmt(fmt, T, H, ksplit, xc);
+}
+
 int xtu_decode_route_shared_ok(int fmt, int mode, int T, int E, int K, int n_group,
                                int n_shared, int H, int I) {
   int ksplit = 0, xc = 0;

@@ -60,6 +60,12 @@ SIGNATURES = {
                               _vp]),
     "xtu_decode_gate_up_routed": (_i, [_i, _vp, _i, _i, _i, _vp, _vp, _vp, _l, _l, _vp, _vp,
                                        _vp, _vp, _vp, _vp, _i, _i, _vp, _f, _f, _f, _vp]),
+    "xtu_stream_max_tile_m": (_i, [_i]),
+    "xtu_stream_gate_up": (_i, [_i, _vp, _i, _vp, _i, _i, _vp, _vp, _vp, _l, _l, _vp, _vp, _vp,
+                                _vp, _vp, _vp, _i, _i, _vp, _f, _f, _f, _vp]),
+    "xtu_stream_down": (_i, [_i, _vp, _i, _i, _vp, _vp, _vp, _l, _l, _vp, _vp, _vp, _vp, _vp,
+                             _vp, _i, _i, _vp, _vp, _vp]),
+    "xtu_decode_gate_up_fast": (_i, [_i, _i, _i]),
     "xtu_gemm_tile_m": (_i, [_i]),
     "xtu_gemm_gate_up": (_i, [_i, _vp, _vp, _i, _i, _vp, _vp, _vp, _l, _l, _vp, _vp, _vp, _vp,
                               _vp, _vp, _i, _vp, _f, _f, _f, _vp]),
@@ -135,6 +141,7 @@ SIGNATURES = {
 _NOT_STATUS = {"xtu_version", "xtu_error_string", "xtu_segment_workspace_bytes",
                "xtu_route_segment_small_max_pairs",
                "xtu_segment_max_tiles", "xtu_gemm_tile_m", "xtu_gemm8_tile_m",
+               "xtu_stream_max_tile_m", "xtu_decode_gate_up_fast",
                "xtu_mx_pair_fits", "xtu_mx_pair_tile_m", "xtu_f8_pair_fits",
                "xtu_f8_pair_tile_m",
                "xtu_decode_down_combine_ok", "xtu_decode_route_shared_ok",

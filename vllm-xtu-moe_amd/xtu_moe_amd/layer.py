@@ -631,6 +631,79 @@ def gemm_tile_m(fmt: int, int8: bool = False, H: int = 0, I: int = 0, W=None,
     return int(_lib.call("xtu_gemm_tile_m", int(fmt)))
 
 
+# Grouped GEMMs of batches that give an expert few rows (xtu_stream_*): the
+# weights stream from HBM at 5-7 TB/s, where the prefill kernels' 128-row
+# tiles wait on one step of weights at a time.  Measured on MI355X (gate/up +
+# down; r = T * K / E rows per expert): MXFP4 (against the triples' kernel)
+# Qwen3-Next r = 40 247 vs 345 us, DeepSeek-V3 r = 25 1213 vs 1380, r = 50
+# 1724 vs 1690; FP8 (against the exact pairs) DeepSeek-V3 r = 22 1960 vs
+# 2090, 128 experts r = 37 121 vs 150, r = 75 192 vs 182; BF16 (against the
+# same products in 128-row tiles) 128 experts r = 62 248 vs 274 (whole layer),
+# r = 125 364 vs 354; NVFP4 (the same) at every r: Qwen3-Next r = 80 546 vs
+# 637.  Tiles of 16 rows hold the weights of up to four
+# workgroups per CU; past a few rows per expert a second tile would read an
+# expert's weights again, and the taller tiles win: Qwen3-Next MXFP4 r = 1.3
+# 104 vs 114 us, r = 6 148 vs 160, r = 14 182 vs 172; DeepSeek-V3 r = 6.5 974
+# vs 965, r = 12.5 1270 vs 1015.
+STREAM_MAX_ROWS = {FMT_MXFP4: 40.0, FMT_FP8: 24.0, FMT_NVFP4: math.inf, FMT_BF16: 90.0}
+STREAM_SHORT_ROWS = 5.0    # rows per expert up to which tiles are 16 rows
+STREAM_TALL_ROWS = 44.0    # ... past which they are 128 (NVFP4, BF16)
+# work items (128-column ones) below which the narrow items of the kernels
+# for small batches fill the chip better: tiny Mixtral BF16 T = 128 (208 items)
+# 32 vs 26 us
+STREAM_MIN_ITEMS = 384
+
+
+def stream_tile_m(fmt: int, T: int, K: int, E: int, NS: int, H: int, I: int) -> int:
+    """Rows per tile of the weight-streaming grouped GEMMs for a batch of T
+    tokens, or 0 where the prefill kernels run it (many rows per expert, few
+    work items, or a prefill kernel chosen by XTU_MXFP4_PREFILL /
+    XTU_FP8_PREFILL)."""
+    fmt = int(fmt)
+    r = T * K / E
+    if fmt not in STREAM_MAX_ROWS or r > STREAM_MAX_ROWS[fmt] or T * H * 2 >= 1 << 31:
+        return 0
+    if fmt == FMT_MXFP4 and os.environ.get(MXFP4_PREFILL_ENV, MXFP4_PREFILL_DEFAULT) != "auto":
+        return 0
+    if fmt == FMT_FP8 and os.environ.get(FP8_PREFILL_ENV, "auto") != "auto":
+        return 0
+    bm = 16 if r <= STREAM_SHORT_ROWS else 64
+    if r > STREAM_TALL_ROWS:
+        bm = int(_lib.call("xtu_stream_max_tile_m", fmt))
+    tiles = min(T * K, E) + T * K // bm + NS * (-(-T // bm))
+    return bm if tiles * (I // 128) >= STREAM_MIN_ITEMS else 0
+
+
+def decode_stream_gate_up(fmt: int, T: int, H: int, I: int, max_tiles: int) -> bool:
+    """Whether a decode batch's gate/up streams in 64-column workgroups
+    (xtu_stream_gate_up): where the decode kernel's workgroups of 16 columns
+    would stage rows piecewise or take several rounds of weights
+    (xtu_decode_gate_up_fast).  Measured on MI355X: DeepSeek-V3 MXFP4 T = 5 / 8
+    / 16 149 / 225 / 366 -> 96 / 139 / 233 us, FP8 T = 3 / 16 132 / 533 -> 119 /
+    433; Qwen3-Next NVFP4 T = 6 / 16 28.5 / 80 -> 23 / 43; 128-expert FP8 T = 16
+    50 -> 43.  Where the fast form holds the decode kernel is the faster one
+    (Qwen3-Next NVFP4 T = 4 19.0 vs 21.8, 128-expert FP8 T = 8 27.9 vs 29.2),
+    and with few work items (tiny Mixtral T = 16: 13.2 vs 13.2)."""
+    return (not _lib.call("xtu_decode_gate_up_fast", int(fmt), int(T), int(H))
+            and max_tiles * (I // 64) >= STREAM_MIN_ITEMS)
+
+
+STREAM_DOWN_MAX_I = 1024   # decode: the down pass streams in wide items up to this K ...
+STREAM_DOWN_MIN_ITEMS = {FMT_MXFP4: 512, FMT_FP8: 512, FMT_NVFP4: 768}   # ... and this many items
+
+
+def decode_stream_down(fmt: int, H: int, I: int, max_tiles: int) -> bool:
+    """Whether a decode batch's down pass takes 128-column workgroups
+    (xtu_stream_down): a short K makes the decode kernel's waves short (four
+    units at I = 512).  Measured on MI355X: Qwen3-Next MXFP4 T = 4 / 8 / 16
+    10.6 / 17.1 / 27.4 -> 8.4 / 10.9 / 17.0 us, NVFP4 T = 6 / 16 14.8 / 28.8 ->
+    13.4 / 22.0 (T = 4: equal, 0.4 us slower per layer),
+    128-expert FP8 (I = 768) T = 4 10.8 -> 10.2, BF16 T = 16 40.3 vs 41.9 (not
+    taken); DeepSeek-V3 (I = 2048) T = 4 41.5 vs 42.4, T = 16 equal."""
+    return (fmt in STREAM_DOWN_MIN_ITEMS and I <= STREAM_DOWN_MAX_I
+            and max_tiles * (H // 128) >= STREAM_DOWN_MIN_ITEMS[fmt])
+
+
 FUSED_DOWN_ENV = "XTU_DECODE_FUSED_DOWN"
 
 
@@ -817,8 +890,9 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
                 router=None, fp8_scales_ok=None):
     """Routed (+shared) experts of one layer; returns out [T, H].
 
-    path: "auto" (decode kernels for T <= 16, grouped GEMMs otherwise),
-    "decode" or "gemm".  int8: INT8-activation x FP4-code ALIGN path (MXFP4):
+    path: "auto" (decode kernels for T <= 16, grouped GEMMs otherwise, either
+    streaming in wider work items where that is faster), or "decode" / "gemm"
+    for the decode / prefill kernels themselves.  int8: INT8-activation x FP4-code ALIGN path (MXFP4):
     True forces it, "auto" applies the reference's token-count gate
     (int8_align_on).
     id_map: int32 [E] applied to topk_ids before bucketing; slot_map: int32
@@ -856,13 +930,18 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
     if int8 == "auto":
         int8 = int8_align_on(T, True)
     int8 = bool(int8)
-    if path == "auto":
+    auto = path == "auto"
+    if auto:
         path = "decode" if (T <= DECODE_MAX_TOKENS and not int8) else "gemm"
     if path == "decode" and T > DECODE_MAX_TOKENS:
         raise ValueError(f"decode path handles at most {DECODE_MAX_TOKENS} tokens")
     # decode: the gate/up and down kernels take the segmentation's 16-row
     # tiles as work slots (every row of a bucket, however many)
-    bm = DECODE_TILE if path == "decode" else gemm_tile_m(fmt, int8, W.H, W.I, W, fp8_scales_ok)
+    stream_bm = 0
+    if auto and path == "gemm" and not int8:
+        stream_bm = stream_tile_m(fmt, T, K, E, NS, H, I)
+    bm = (DECODE_TILE if path == "decode"
+          else stream_bm or gemm_tile_m(fmt, int8, W.H, W.I, W, fp8_scales_ok))
     seg = segmentation(T, K, E, NS, bm, dev, st)
     odt = out_dtype if out is None else out.dtype
     max_active = min(E, T * K) + NS
@@ -971,6 +1050,12 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
                       _p(W.gs13), 0, 0, _p(slot_map), _p(seg.sorted_tok), _p(seg.seg_start),
                       _p(seg.tile_expert), _p(seg.tile_row0), _p(seg.n_tiles), max_dt, NS,
                       _p(act), lim, al, be, st)
+        elif auto and decode_stream_gate_up(fmt, T, H, I, max_dt):
+            lo, hi = seg.tile_range_ptrs(0, E + NS)
+            _lib.call("xtu_stream_gate_up", fmt, _p(x), T, _p(seg.sorted_tok), H, I, _p(W.w13),
+                      _p(W.s13), _p(W.gs13), 0, 0, _p(slot_map), _p(seg.seg_start),
+                      _p(seg.tile_expert), _p(seg.tile_row0), lo, hi, seg.bm, max_dt, _p(act),
+                      lim, al, be, st)
         else:
             _lib.call("xtu_decode_gate_up", fmt, _p(x), T, H, I, _p(W.w13), _p(W.s13),
                       _p(W.gs13), 0, 0, _p(slot_map), _p(seg.sorted_tok), _p(seg.seg_start),
@@ -989,10 +1074,17 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
         if (os.environ.get(DOWN_BY_PAIR_ENV, "1") != "0" and K in COMBINE_BY_PAIR_K
                 and NS <= 2 and out.dtype in (torch.bfloat16, torch.float32)):
             # y rows in flat pair order: the combine's loads need no inv first
-            _lib.call("xtu_decode_down_by_pair", fmt, _p(act), T, H, I, _p(W.w2), _p(W.s2),
-                      _p(W.gs2), 0, 0, _p(slot_map), _p(seg.seg_start), _p(seg.tile_expert),
-                      _p(seg.tile_row0), _p(seg.n_tiles), max_dt, _p(seg.sorted_pair), _p(y),
-                      st)
+            if auto and decode_stream_down(fmt, H, I, max_dt):
+                lo, hi = seg.tile_range_ptrs(0, E + NS)
+                _lib.call("xtu_stream_down", fmt, _p(act), H, I, _p(W.w2), _p(W.s2), _p(W.gs2), 0,
+                          0, _p(slot_map), _p(seg.seg_start), _p(seg.tile_expert),
+                          _p(seg.tile_row0), lo, hi, seg.bm, max_dt, _p(seg.sorted_pair), _p(y),
+                          st)
+            else:
+                _lib.call("xtu_decode_down_by_pair", fmt, _p(act), T, H, I, _p(W.w2), _p(W.s2),
+                          _p(W.gs2), 0, 0, _p(slot_map), _p(seg.seg_start), _p(seg.tile_expert),
+                          _p(seg.tile_row0), _p(seg.n_tiles), max_dt, _p(seg.sorted_pair), _p(y),
+                          st)
             _lib.call("xtu_combine_by_pair", _p(y), _p(seg.inv), _p(wts),
                       _p(seg.seg_start) + 4 * (seg.E + seg.NS), T, K, NS, H, _p(out),
                       int(out.dtype == torch.bfloat16), st)
@@ -1004,7 +1096,8 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
         y = _buf("y", (max(A, 1), H), torch.float32, dev, st)
         expert_pass(x, seg, W, 0, E + NS, y, slot_map=slot_map, int8=int8,
                     swiglu_limit=swiglu_limit, swiglu_alpha=swiglu_alpha,
-                    swiglu_beta=swiglu_beta, stream=st, fp8_scales_ok=fp8_scales_ok)
+                    swiglu_beta=swiglu_beta, stream=st, fp8_scales_ok=fp8_scales_ok,
+                    stream_bm=stream_bm)
     combine(seg, y, wts, out, stream=st)
     return (out, seg) if return_seg else out
 
@@ -1023,11 +1116,12 @@ def act_quant_fused() -> bool:
 
 def expert_pass(x, seg, W: ExpertWeights, b0: int, b1: int, y, *, slot_map=None, int8=False,
                 swiglu_limit=0.0, swiglu_alpha=1.0, swiglu_beta=0.0, stream=None,
-                fp8_scales_ok=None):
+                fp8_scales_ok=None, stream_bm=0):
     """Grouped gate/up (+ SwiGLU-clamp) and down GEMMs for the sorted pairs of
     buckets [b0, b1), weights of bucket b at slot slot_map[b] of W (identity
     without a map); writes their fp32 rows of y [A, H].  The segmentation's
-    tile height must be gemm_tile_m(..., W, fp8_scales_ok)'s."""
+    tile height must be gemm_tile_m(..., W, fp8_scales_ok)'s, or stream_bm
+    (stream_tile_m) where that is set: the weight-streaming kernels."""
     T, H = x.shape
     I = W.I
     A = seg.A
@@ -1072,6 +1166,15 @@ def expert_pass(x, seg, W: ExpertWeights, b0: int, b1: int, y, *, slot_map=None,
                   _p(seg.tile_row0), lo, hi, seg.max_tiles, seg.bm, _p(y), 0.0, 1.0, 0.0, st)
         return
     fmt = W.fmt
+    if stream_bm:
+        _lib.call("xtu_stream_gate_up", fmt, _p(x), T, _p(seg.sorted_tok), H, I, _p(W.w13),
+                  _p(W.s13), _p(W.gs13), 0, 0, _p(slot_map), _p(seg.seg_start),
+                  _p(seg.tile_expert), _p(seg.tile_row0), lo, hi, stream_bm, seg.max_tiles,
+                  _p(act), lim, al, be, st)
+        _lib.call("xtu_stream_down", fmt, _p(act), H, I, _p(W.w2), _p(W.s2), _p(W.gs2), 0, 0,
+                  _p(slot_map), _p(seg.seg_start), _p(seg.tile_expert), _p(seg.tile_row0), lo, hi,
+                  stream_bm, seg.max_tiles, 0, _p(y), st)
+        return
     if fp8_pair32_use(W, fp8_scales_ok):
         # exact pairs, interleaved, on the FP8 32x32x64 kernel (block scales
         # applied by accumulator rescaling)
