@@ -42,11 +42,15 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
   return (uint16_t)(u >> 16);
 }
 
-// e4m3fn byte -> fp32 (normal: exponent rebias by +120; subnormal m * 2^-9).
+// e4m3fn byte -> fp32: the exponent and mantissa bits moved into an fp32's
+// read as 2^(e - 127) (1 + m/8), or m 2^-129 for e = 0 (fp32 subnormals are
+// kept), so one multiply by 2^120 rebiases both, exactly and without a branch
+// (a select on e = 0 compiles to exec-mask branches, 16 of them per four
+// super-blocks of two NVFP4 panels: 1172 -> 754 instructions with the byte
+// permute of fp4x8_to_bf16_mul).
 __device__ __forceinline__ float e4m3_to_f32(uint32_t b) {
-  const uint32_t e = (b >> 3) & 15u, m = b & 7u;
-  float v = (e == 0) ? (float)m * 1.953125e-03f : __uint_as_float(((e + 120u) << 23) | (m << 20));
-  return (b & 0x80u) ? -v : v;
+  const float v = __uint_as_float((b & 0x7fu) << 20) * 1.329227995784915873e+36f;
+  return __uint_as_float(__float_as_uint(v) | ((b & 0x80u) << 24));
 }
 
 // e8m0 byte -> 2^(b-127) as fp32 (b = 0 gives 2^-127, a subnormal; b = 255 inf).
@@ -137,7 +141,7 @@ __device__ __forceinline__ void fp4x8_to_bf16_mul(uint32_t w, float scale, uint3
   for (int i = 0; i < 4; ++i) {
     const uint32_t lo = __float_as_uint(vv[i][0] * scale);
     const uint32_t hi = __float_as_uint(vv[i][1] * scale);
-    out[i] = (lo >> 16) | (hi & 0xffff0000u);
+    out[i] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);   // high halves: hi:lo
   }
 }
 
