@@ -314,6 +314,23 @@ hipError_t xtu_stream_down(int fmt, const void* act, int H, int I, const void* w
                            const int32_t* tile_lo, const int32_t* tile_hi, int bm, int max_tiles,
                            const int32_t* sorted_pair, float* y, hipStream_t stream);
 int xtu_decode_gate_up_fast(int fmt, int T, int H);
+/* The INT8 ALIGN products (xtu_i8_gemm_gate_up / _down below, bit for bit)
+ * read from the MXFP4 codes and scales themselves, expanded in registers
+ * (half the bytes of the expanded planes): a8 / crow from xtu_i8_quant_rows,
+ * emin from xtu_i8_prepare, tiles of at most 128 rows. */
+hipError_t xtu_stream_i8_gate_up(const int8_t* a8, const int32_t* crow, int T,
+                                 const int32_t* sorted_tok, int H, int I, const void* w13,
+                                 const void* s13, const uint8_t* emin13, const int32_t* slot_map,
+                                 const int32_t* seg_start, const int32_t* tile_expert,
+                                 const int32_t* tile_row0, const int32_t* tile_lo,
+                                 const int32_t* tile_hi, int bm, int max_tiles, void* act,
+                                 float limit, float alpha, float beta, hipStream_t stream);
+hipError_t xtu_stream_i8_down(const int8_t* a8, const int32_t* crow, int H, int I, const void* w2,
+                              const void* s2, const uint8_t* emin2, const int32_t* slot_map,
+                              const int32_t* seg_start, const int32_t* tile_expert,
+                              const int32_t* tile_row0, const int32_t* tile_lo,
+                              const int32_t* tile_hi, int bm, int max_tiles, float* y,
+                              hipStream_t stream);
 
 /* ------------------------------------------------ grouped GEMM (prefill) path
  * Replaces _gate_up_kernel / _down_kernel (vllm_xiaotu_moe/gpu_prefill.py:

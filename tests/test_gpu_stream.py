@@ -76,7 +76,8 @@ def test_layer_takes_them(fmt, T):
     ids, wts = random_routing(T, K, E, seed=T, invalid_frac=0.05, zero_frac=0.05)
     x = torch.randn((T, H), generator=torch.Generator().manual_seed(T)).to(torch.bfloat16)
     if T > L.DECODE_MAX_TOKENS:
-        assert L.stream_tile_m(fmt, T, K, E, NS, H, I) == (16 if T == 40 else 64)
+        want = {F.FMT_FP8: 64, F.FMT_BF16: 128}.get(fmt, 16 if T == 40 else 64)
+        assert L.stream_tile_m(fmt, T, K, E, NS, H, I) == want
     else:
         n = L.decode_max_tiles(T * (K + NS), min(E, T * K) + NS)
         assert L.decode_stream_gate_up(fmt, T, H, I, n) == (fmt != F.FMT_BF16)
@@ -93,3 +94,63 @@ def test_layer_takes_them(fmt, T):
     torch.cuda.synchronize()
     ref = oracle_layer(fmt, dense_to_numpy(fmt, d), bf16_tensor_to_bits(x), ids, wts, E, NS, H, I)
     check_close(out.cpu().numpy(), ref, bf16_out=False, what=f"stream layer fmt={fmt} T={T}")
+
+
+@pytest.mark.parametrize("bm", [16, 64, 128])
+@pytest.mark.parametrize("H,I", [(256, 128), (768, 384)])
+def test_int8_rows_equal_the_expanded_planes(bm, H, I):
+    """Codes expanded in registers: bitwise the integer GEMM over the expanded
+    planes, with scale spreads of 0..3 and rows marked for the fallback (their
+    columns are zero sums in both)."""
+    E = len(ROWS)
+    fmt = F.FMT_MXFP4
+    ids = np.repeat(np.arange(E, dtype=np.int32), ROWS)
+    rng = np.random.default_rng(bm + I)
+    rng.shuffle(ids)
+    T = len(ids)
+    d, _ = _weights(fmt, E, 0, H, I, seed=H)
+    for k in ("s13", "s2"):   # spread 0..3 per row, a few rows past it
+        s = d[k].to(torch.int32)
+        s = 120 + torch.randint(0, 4, s.shape, generator=torch.Generator().manual_seed(3))
+        s[:, 5::37, 0] = 131
+        d[k] = s.to(torch.uint8)
+    W = ExpertWeights.from_dense(fmt, d["w13"], d["s13"], d["w2"], d["s2"], n_shared=0,
+                                 device="cuda")
+    w13_8, em13, w2_8, em2 = W.int8_planes()
+    x = torch.randn((T, H), generator=torch.Generator().manual_seed(T)).to(torch.bfloat16).cuda()
+    idd = torch.from_numpy(ids[:, None].copy()).cuda()
+    wd = torch.ones((T, 1), device="cuda")
+    st = _stream()
+    dev = x.device
+    a8 = torch.empty((T, H), dtype=torch.int8, device=dev)
+    cr = torch.empty(T, dtype=torch.int32, device=dev)
+    _lib.call("xtu_i8_quant_rows", _p(x), T, H, _p(a8), _p(cr), st)
+    acts, ys = [], []
+    for b in (128, bm):
+        seg = L.segmentation(T, 1, E, 0, b, dev)
+        seg.run(idd, wd)
+        lo, hi = seg.tile_range_ptrs(0, E)
+        act = torch.full((T, I), float("nan"), dtype=torch.bfloat16, device=dev)
+        a8a = torch.empty((T, I), dtype=torch.int8, device=dev)
+        cra = torch.empty(T, dtype=torch.int32, device=dev)
+        y = torch.full((T, H), float("nan"), device=dev)
+        tiles = (_p(seg.seg_start), _p(seg.tile_expert), _p(seg.tile_row0), lo, hi)
+        if not acts:
+            _lib.call("xtu_i8_gemm_gate_up", _p(a8), _p(cr), _p(seg.sorted_tok), H, I, _p(w13_8),
+                      _p(em13), 0, *tiles, seg.max_tiles, _p(act), 0, 2.0, 1.0, 0.0, st)
+        else:
+            _lib.call("xtu_stream_i8_gate_up", _p(a8), _p(cr), T, _p(seg.sorted_tok), H, I,
+                      _p(W.w13), _p(W.s13), _p(em13), 0, *tiles, b, seg.max_tiles, _p(act), 2.0,
+                      1.0, 0.0, st)
+        _lib.call("xtu_i8_quant_rows", _p(act), T, I, _p(a8a), _p(cra), st)
+        if not acts:
+            _lib.call("xtu_i8_gemm_down", _p(a8a), _p(cra), H, I, _p(w2_8), _p(em2), 0, *tiles,
+                      seg.max_tiles, _p(y), 0, st)
+        else:
+            _lib.call("xtu_stream_i8_down", _p(a8a), _p(cra), H, I, _p(W.w2), _p(W.s2), _p(em2),
+                      0, *tiles, b, seg.max_tiles, _p(y), st)
+        acts.append(act)
+        ys.append(y)
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(ys[0]).all())
+    assert torch.equal(acts[0], acts[1]) and torch.equal(ys[0], ys[1])

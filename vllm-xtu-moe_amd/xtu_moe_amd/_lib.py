@@ -66,6 +66,10 @@ SIGNATURES = {
     "xtu_stream_down": (_i, [_i, _vp, _i, _i, _vp, _vp, _vp, _l, _l, _vp, _vp, _vp, _vp, _vp,
                              _vp, _i, _i, _vp, _vp, _vp]),
     "xtu_decode_gate_up_fast": (_i, [_i, _i, _i]),
+    "xtu_stream_i8_gate_up": (_i, [_vp, _vp, _i, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                   _vp, _vp, _i, _i, _vp, _f, _f, _f, _vp]),
+    "xtu_stream_i8_down": (_i, [_vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i,
+                                _i, _vp, _vp]),
     "xtu_gemm_tile_m": (_i, [_i]),
     "xtu_gemm_gate_up": (_i, [_i, _vp, _vp, _i, _i, _vp, _vp, _vp, _l, _l, _vp, _vp, _vp, _vp,
                               _vp, _vp, _i, _vp, _f, _f, _f, _vp]),

@@ -633,25 +633,28 @@ def gemm_tile_m(fmt: int, int8: bool = False, H: int = 0, I: int = 0, W=None,
 
 # Grouped GEMMs of batches that give an expert few rows (xtu_stream_*): the
 # weights stream from HBM at 5-7 TB/s, where the prefill kernels' 128-row
-# tiles wait on one step of weights at a time.  Measured on MI355X (gate/up +
-# down; r = T * K / E rows per expert): MXFP4 (against the triples' kernel)
-# Qwen3-Next r = 40 247 vs 345 us, DeepSeek-V3 r = 25 1213 vs 1380, r = 50
-# 1724 vs 1690; FP8 (against the exact pairs) DeepSeek-V3 r = 22 1960 vs
-# 2090, 128 experts r = 37 121 vs 150, r = 75 192 vs 182; BF16 (against the
-# same products in 128-row tiles) 128 experts r = 62 248 vs 274 (whole layer),
-# r = 125 364 vs 354; NVFP4 (the same) at every r: Qwen3-Next r = 80 546 vs
-# 637.  Tiles of 16 rows hold the weights of up to four
-# workgroups per CU; past a few rows per expert a second tile would read an
-# expert's weights again, and the taller tiles win: Qwen3-Next MXFP4 r = 1.3
-# 104 vs 114 us, r = 6 148 vs 160, r = 14 182 vs 172; DeepSeek-V3 r = 6.5 974
-# vs 965, r = 12.5 1270 vs 1015.
-STREAM_MAX_ROWS = {FMT_MXFP4: 40.0, FMT_FP8: 24.0, FMT_NVFP4: math.inf, FMT_BF16: 90.0}
-STREAM_SHORT_ROWS = 5.0    # rows per expert up to which tiles are 16 rows
-STREAM_TALL_ROWS = 44.0    # ... past which they are 128 (NVFP4, BF16)
-# work items (128-column ones) below which the narrow items of the kernels
-# for small batches fill the chip better: tiny Mixtral BF16 T = 128 (208 items)
-# 32 vs 26 us
-STREAM_MIN_ITEMS = 384
+# tiles wait on one step of weights at a time.  Whole layers on MI355X by
+# rows per expert r = T * K / E, against the prefill kernels: MXFP4 DeepSeek-V3
+# r = 6 / 25 / 44 / 50 985 / 1213 / 1622 / 1797 vs 1205 / 1420 / 1683 / 1780 us,
+# Qwen3-Next r = 49 334 vs 414; FP8 DeepSeek-V3 r = 31 / 37 2147 / 2303 vs 2244 /
+# 2356, 128 experts r = 50 / 62 164 / 200 vs 183 / 205; BF16 128 experts r = 62 /
+# 100 / 125 248 / 294 / 364 vs 276 / 319 / 354; NVFP4 Qwen3-Next r = 21 / 80 /
+# 160 at every size (289 / 563 / 1074 vs 431 / 662 / 1220).
+STREAM_MAX_ROWS = {FMT_MXFP4: 46.0, FMT_FP8: 40.0, FMT_NVFP4: math.inf, FMT_BF16: 110.0}
+# Tile heights.  Up to SHORT rows per expert 16-row tiles (their LDS stage and
+# registers let four workgroups share a CU; a second tile of an expert reads
+# its weights again): MXFP4 r = 2.9 / 4.9 / 6.2 161 / 166 / 1010 vs 170 / 178 /
+# 985 us on 64-row ones (the last DeepSeek-V3), NVFP4 r = 4.9 / 7.8 / 11.7 193 /
+# 204 / 229 vs 209 / 210 / 226, FP8 r = 1.9 1407 vs 1388 (never), BF16 r = 5 195 vs
+# 194 (never).  Past TALL 128-row tiles: NVFP4 r = 59 / 68 509 / 563 vs 464 / 566;
+# BF16 r = 5 / 50 194 / 235 vs 194 / 257 (always).
+STREAM_SHORT_ROWS = {FMT_MXFP4: 5.0, FMT_NVFP4: 10.0}
+STREAM_TALL_ROWS = {FMT_NVFP4: 66.0, FMT_BF16: 0.0}
+STREAM_I8_TALL_ROWS = 66.0   # int8 activations: r = 59 / 80 446 / 526 vs 400 / 587 us
+# BF16 work items (128 columns) below which the prefill kernels' narrow items
+# for small batches fill the chip better: tiny Mixtral T = 128 (176 items) 36
+# vs 41 us.  The other formats have no such items: tiny MXFP4 58 vs 40.
+STREAM_BF16_MIN_ITEMS = 384
 
 
 def stream_tile_m(fmt: int, T: int, K: int, E: int, NS: int, H: int, I: int) -> int:
@@ -667,11 +670,32 @@ def stream_tile_m(fmt: int, T: int, K: int, E: int, NS: int, H: int, I: int) -> 
         return 0
     if fmt == FMT_FP8 and os.environ.get(FP8_PREFILL_ENV, "auto") != "auto":
         return 0
-    bm = 16 if r <= STREAM_SHORT_ROWS else 64
-    if r > STREAM_TALL_ROWS:
-        bm = int(_lib.call("xtu_stream_max_tile_m", fmt))
-    tiles = min(T * K, E) + T * K // bm + NS * (-(-T // bm))
-    return bm if tiles * (I // 128) >= STREAM_MIN_ITEMS else 0
+    bm = 16 if r <= STREAM_SHORT_ROWS.get(fmt, 0.0) else 64
+    if r > STREAM_TALL_ROWS.get(fmt, math.inf):
+        bm = 128
+    if fmt == FMT_BF16:
+        tiles = min(T * K, E) + T * K // bm + NS * (-(-T // bm))
+        if tiles * (I // 128) < STREAM_BF16_MIN_ITEMS:
+            return 0
+    return bm
+
+
+def stream_i8_tile_m(T: int, K: int, E: int, H: int) -> int:
+    """stream_tile_m for the INT8 ALIGN path (xtu_stream_i8_*, bitwise the
+    same outputs): the MXFP4 codes expanded in registers are half the bytes
+    of the expanded planes, at every size measured.  Whole layer on MI355X:
+    Qwen3-Next T = 160 / 1000 / 3000 / 8192 318 / 367 / 503 / 1053 -> 198 / 252 /
+    400 / 1007 us, DeepSeek-V3 T = 500 / 4096 1916 / 3888 -> 1207 / 3491.
+    tiny (8 experts) T = 160 / 4000 65 / 188 -> 44 / 176."""
+    r = T * K / E
+    if T * H >= 1 << 31:
+        return 0
+    # a decode batch (int8 forced below its token gate) has one tile per expert
+    # at either height and keeps the integer GEMMs' own
+    return 64 if r <= STREAM_I8_TALL_ROWS and T > DECODE_MAX_TOKENS else 128
+
+
+DECODE_STREAM_MIN_ITEMS = 384
 
 
 def decode_stream_gate_up(fmt: int, T: int, H: int, I: int, max_tiles: int) -> bool:
@@ -685,7 +709,7 @@ def decode_stream_gate_up(fmt: int, T: int, H: int, I: int, max_tiles: int) -> b
     (Qwen3-Next NVFP4 T = 4 19.0 vs 21.8, 128-expert FP8 T = 8 27.9 vs 29.2),
     and with few work items (tiny Mixtral T = 16: 13.2 vs 13.2)."""
     return (not _lib.call("xtu_decode_gate_up_fast", int(fmt), int(T), int(H))
-            and max_tiles * (I // 64) >= STREAM_MIN_ITEMS)
+            and max_tiles * (I // 64) >= DECODE_STREAM_MIN_ITEMS)
 
 
 STREAM_DOWN_MAX_I = 1024   # decode: the down pass streams in wide items up to this K ...
@@ -938,8 +962,9 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
     # decode: the gate/up and down kernels take the segmentation's 16-row
     # tiles as work slots (every row of a bucket, however many)
     stream_bm = 0
-    if auto and path == "gemm" and not int8:
-        stream_bm = stream_tile_m(fmt, T, K, E, NS, H, I)
+    if auto and path == "gemm":
+        stream_bm = (stream_i8_tile_m(T, K, E, H) if int8
+                     else stream_tile_m(fmt, T, K, E, NS, H, I))
     bm = (DECODE_TILE if path == "decode"
           else stream_bm or gemm_tile_m(fmt, int8, W.H, W.I, W, fp8_scales_ok))
     seg = segmentation(T, K, E, NS, bm, dev, st)
@@ -1141,9 +1166,16 @@ def expert_pass(x, seg, W: ExpertWeights, b0: int, b1: int, y, *, slot_map=None,
         _lib.call("xtu_i8_quant_rows", _p(x), T, H, _p(a8x), _p(crx), st)
         fb = W.int8_fallback_cols()
         emm13, emm2 = W.int8_emin_min()
-        _lib.call("xtu_i8_gemm_gate_up", _p(a8x), _p(crx), _p(seg.sorted_tok), H, I, _p(w13_8),
-                  _p(emin13), _p(slot_map), _p(seg.seg_start), _p(seg.tile_expert),
-                  _p(seg.tile_row0), lo, hi, seg.max_tiles, _p(act), 0, lim, al, be, st)
+        if stream_bm:
+            _lib.call("xtu_stream_i8_gate_up", _p(a8x), _p(crx), T, _p(seg.sorted_tok), H, I,
+                      _p(W.w13), _p(W.s13), _p(emin13), _p(slot_map), _p(seg.seg_start),
+                      _p(seg.tile_expert), _p(seg.tile_row0), lo, hi, stream_bm, seg.max_tiles,
+                      _p(act), lim, al, be, st)
+        else:
+            _lib.call("xtu_i8_gemm_gate_up", _p(a8x), _p(crx), _p(seg.sorted_tok), H, I,
+                      _p(w13_8), _p(emin13), _p(slot_map), _p(seg.seg_start),
+                      _p(seg.tile_expert), _p(seg.tile_row0), lo, hi, seg.max_tiles, _p(act), 0,
+                      lim, al, be, st)
         if fb is not None:   # marked weight rows: their columns in fp32
             _lib.call("xtu_i8_fallback", 1, _p(x), _p(seg.sorted_tok), H, I, _p(W.w13),
                       _p(W.s13), _p(slot_map), _p(seg.seg_start), _p(seg.tile_expert),
@@ -1154,9 +1186,14 @@ def expert_pass(x, seg, W: ExpertWeights, b0: int, b1: int, y, *, slot_map=None,
                   _p(W.w13), _p(W.s13), _p(slot_map), _p(seg.seg_start), _p(seg.tile_expert),
                   _p(seg.tile_row0), lo, hi, seg.max_tiles, seg.bm, _p(act), lim, al, be, st)
         _lib.call("xtu_i8_quant_rows", _p(act), A, I, _p(a8a), _p(cra), st)
-        _lib.call("xtu_i8_gemm_down", _p(a8a), _p(cra), H, I, _p(w2_8), _p(emin2), _p(slot_map),
-                  _p(seg.seg_start), _p(seg.tile_expert), _p(seg.tile_row0), lo, hi,
-                  seg.max_tiles, _p(y), 0, st)
+        if stream_bm:
+            _lib.call("xtu_stream_i8_down", _p(a8a), _p(cra), H, I, _p(W.w2), _p(W.s2),
+                      _p(emin2), _p(slot_map), _p(seg.seg_start), _p(seg.tile_expert),
+                      _p(seg.tile_row0), lo, hi, stream_bm, seg.max_tiles, _p(y), st)
+        else:
+            _lib.call("xtu_i8_gemm_down", _p(a8a), _p(cra), H, I, _p(w2_8), _p(emin2),
+                      _p(slot_map), _p(seg.seg_start), _p(seg.tile_expert), _p(seg.tile_row0),
+                      lo, hi, seg.max_tiles, _p(y), 0, st)
         if fb is not None:
             _lib.call("xtu_i8_fallback", 0, _p(act), 0, H, I, _p(W.w2), _p(W.s2), _p(slot_map),
                       _p(seg.seg_start), _p(seg.tile_expert), _p(seg.tile_row0), lo, hi,
