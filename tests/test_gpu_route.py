@@ -195,6 +195,39 @@ def test_wave_routed_small_batch_bit_exact(T, E, K, mode):
     np.testing.assert_array_equal(seg.sorted_pair.cpu().numpy()[: seg.A], ref["sorted_pair"])
 
 
+@pytest.mark.parametrize("T", [1, 5, 16, 33, 4096])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_two_experts_per_lane_router_bit_exact(T, mode):
+    """E = 128: ties, -0 / +0 and K = 8, on the one-launch router (T <= 16) and
+    the batch one."""
+    E, K = 128, 8
+    rng = np.random.default_rng(T + mode)
+    logits = rng.standard_normal((T, E)).astype(np.float32)
+    logits[::2] = np.round(logits[::2] * 2) / 2
+    logits[0, 3::7] = -0.0
+    bias = (rng.standard_normal(E) * 0.05).astype(np.float32) if mode else None
+    dev = torch.device("cuda")
+    tl = torch.from_numpy(logits).to(dev)
+    tb = None if bias is None else torch.from_numpy(bias).to(dev)
+    if mode == 0:
+        rids, rwts = oracle.route_softmax_topk(logits, K)
+    else:
+        rids, rwts = oracle.route_grouped_sigmoid(logits, bias, 8, 4, K, 2.5)
+    kw = dict(n_group=8, topk_group=4, routed_scaling_factor=2.5, bias=tb) if mode else {}
+    wts, ids = L.route(tl, top_k=K, scoring="sigmoid" if mode else "softmax", **kw)
+    got = [(ids, wts)]
+    if T <= 16:
+        seg = L.segmentation(T, K, E, 0, 16, dev)
+        i2, w2 = torch.empty_like(ids), torch.empty_like(wts)
+        kw2 = dict(n_group=8, topk_group=4, routed_scaling=2.5, bias=tb) if mode else {}
+        seg.run_small(mode, i2, w2, logits=tl, **kw2)
+        got.append((i2, w2))
+    torch.cuda.synchronize()
+    for i, w in got:
+        np.testing.assert_array_equal(i.cpu().numpy(), rids)
+        np.testing.assert_array_equal(w.cpu().numpy().view(np.uint32), rwts.view(np.uint32))
+
+
 @pytest.mark.parametrize("T,K,E,NS", [(14564, 8, 256, 1), (14563, 8, 255, 1), (30000, 10, 512, 1),
                                       (114, 8, 256, 1), (113, 9, 9, 0)])
 def test_segmentation_block_round_edges(T, K, E, NS):

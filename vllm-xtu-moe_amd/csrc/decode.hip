@@ -161,7 +161,9 @@ void launch_route_gate_up_xc(int mode, int epl, dim3 grid, int bd, size_t lds,
     else
       decode_route_gate_up_kernel<FMT, 1, 8, XC><<<grid, bd, lds, stream>>>(ra, a, act_sh, n_sh, skip);
   } else {
-    if (epl == 4)
+    if (epl == 2)
+      decode_route_gate_up_kernel<FMT, 0, 2, XC><<<grid, bd, lds, stream>>>(ra, a, act_sh, n_sh, skip);
+    else if (epl == 4)
       decode_route_gate_up_kernel<FMT, 0, 4, XC><<<grid, bd, lds, stream>>>(ra, a, act_sh, n_sh, skip);
     else
       decode_route_gate_up_kernel<FMT, 0, 8, XC><<<grid, bd, lds, stream>>>(ra, a, act_sh, n_sh, skip);
@@ -303,7 +305,8 @@ int xtu_decode_route_shared_ok(int fmt, int mode, int T, int E, int K, int n_gro
   r.renorm = 1;
   static const float probe[4] = {0.f, 0.f, 0.f, 0.f};   // a 16-byte-aligned row stands in
   r.logits = probe;
-  return tiny::tiny_epl(r, mode) != 0;
+  const int epl = tiny::tiny_epl(r, mode);
+  return epl != 0 && epl != 2;   // E = 128 has no instantiation here
 }
 
 hipError_t xtu_decode_route_shared(
@@ -358,7 +361,8 @@ int xtu_decode_route_gate_up_ok(int fmt, int mode, int T, int E, int K, int n_gr
   r.renorm = 1;
   static const float probe[4] = {0.f, 0.f, 0.f, 0.f};   // a 16-byte-aligned row stands in
   r.logits = probe;
-  return tiny::tiny_epl(r, mode) != 0;
+  const int epl = tiny::tiny_epl(r, mode);
+  return epl != 0 && (epl != 2 || mode == 0);   // E = 128: softmax only
 }
 
 hipError_t xtu_decode_route_gate_up(

@@ -371,6 +371,7 @@ int xtu_decode_layer_barrier_words(void) { return kBarWords; }
 int xtu_decode_layer_ok(int fmt, int mode, int T, int E, int K, int n_group, int n_shared,
                         int H, int I) {
   if (!xtu_decode_route_gate_up_ok(fmt, mode, T, E, K, n_group, n_shared, H, I)) return 0;
+  if (mode != 2 && E / kWave != 4 && E / kWave != 8) return 0;   // no two-experts-a-lane form
   int ksplit = 0, xc = 0, ks = 0, ppb = 0, nper = 0;
   bool ok = false;
   switch (fmt) {

@@ -42,7 +42,7 @@ struct SmallArgs {
 };
 
 // ---------------------------------------------------------------------------
-// Tiny batches (at most 64 pairs; routing for E = 64 * EPL, EPL = 4 or 8): one
+// Tiny batches (at most 64 pairs; routing for E = 64 * EPL, EPL = 2, 4 or 8): one
 // wave routes one token with no workgroup barrier.  Lane l holds experts
 // [l*EPL, (l+1)*EPL) and sorts them by (score desc, index asc) once; the K
 // choices are taken in K rounds of a wave-wide maximum of the lanes' first
@@ -116,7 +116,7 @@ __device__ __forceinline__ void cas_desc(uint64_t& a, uint64_t& b) {
 }
 
 // Descending sort of EPL words in registers: the optimal networks for 4 and
-// 8 (5 and 19 compare-exchanges), odd-even transposition otherwise.
+// 8 (5 and 19 compare-exchanges), odd-even transposition otherwise (2: one).
 template <int EPL>
 __device__ __forceinline__ void sort_desc(uint64_t (&c)[EPL]) {
   if constexpr (EPL != 4 && EPL != 8) {
@@ -148,13 +148,15 @@ __device__ void route_token_wave(const float* __restrict__ l, const float* __res
   const int e0 = lane * EPL;
   float x[EPL], bi[EPL], ws[EPL], sc[EPL];
   uint32_t key[EPL];
+  constexpr int VL = EPL < 4 ? EPL : 4;   // scores per load
+  typedef float vec_t __attribute__((ext_vector_type(VL)));
 #pragma unroll
-  for (int j = 0; j < EPL; j += 4) {
-    const f32x4_t v = *reinterpret_cast<const f32x4_t*>(l + e0 + j);
-    f32x4_t bv = {0.f, 0.f, 0.f, 0.f};
-    if (MODE == 1 && bias) bv = *reinterpret_cast<const f32x4_t*>(bias + e0 + j);
+  for (int j = 0; j < EPL; j += VL) {
+    const vec_t v = *reinterpret_cast<const vec_t*>(l + e0 + j);
+    vec_t bv = 0.f;
+    if (MODE == 1 && bias) bv = *reinterpret_cast<const vec_t*>(bias + e0 + j);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < VL; ++q) {
       x[j + q] = v[q];
       bi[j + q] = bv[q];
     }
@@ -417,12 +419,12 @@ __device__ void route_segment_block(const SmallArgs& a, TinySmem& g) {
 }
 
 // Experts per lane of route_token_wave for this router (0: outside its
-// envelope): E = 256 or 512, whole lanes per group, renormalised softmax,
+// envelope): E = 128, 256 or 512, whole lanes per group, renormalised softmax,
 // 16-byte-aligned logit and bias rows.
 __host__ inline int wave_epl(int mode, int E, int n_group, int renorm, const float* logits,
                              const float* bias) {
   const int epl = E / kWave;
-  if (E % kWave != 0 || (epl != 4 && epl != 8)) return 0;
+  if (E % kWave != 0 || (epl != 2 && epl != 4 && epl != 8)) return 0;
   if (reinterpret_cast<uintptr_t>(logits) % 16 != 0 ||
       (bias && reinterpret_cast<uintptr_t>(bias) % 16 != 0))
     return 0;
