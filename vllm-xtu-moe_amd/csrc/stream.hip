@@ -33,8 +33,14 @@
 //   Qwen3-Next MXFP4 T = 300    252 -> 160
 //   DeepSeek-V3 MXFP4 T = 209  1204 -> 965 (6.2 TB/s)
 //   DeepSeek-V3 MXFP4 T = 16 gate/up 366 -> 233 (6.9 TB/s)
-//   DeepSeek-V3 FP8 T = 32      (gate/up 7.0 TB/s)
+//   DeepSeek-V3 FP8 T = 32      1030 (7.0 TB/s)
 //   128-expert FP8 T = 64       132 -> 91
+//   Qwen3-Next NVFP4 T = 4096   637 -> 500 (with the branch-free scales)
+//   Qwen3-Next int8 T = 1000    339 -> 230 (whole layer 367 -> 255)
+// Past some tens of rows per expert the LDS reads of the rows, the
+// dequantisation and the MFMAs share the time about evenly (NVFP4 T = 4096:
+// LDS 40%, VALU 35%, MFMA 31% busy at two waves per SIMD); int8 is bound by
+// the expansion's VALU work (68% busy at T = 1000).
 #include <type_traits>
 
 #include "weight_format.hpp"

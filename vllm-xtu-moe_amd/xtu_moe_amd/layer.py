@@ -555,6 +555,7 @@ def fp8_pair32_use(W, scales_ok=None) -> bool:
     return W.fp8_scales_bounded()
 
 
+# Prefill (many rows per expert; stream_tile_m has the rest under "auto").
 # "auto": the 32x32x64 MXFP4 kernel on activation triples (fp6/fp6/fp4
 # pieces, double-rate MFMA) where it takes the shape, else the bf16-operand
 # kernels; "tri" the same; "pair" exact e4m3 pairs (the 32x32x64 kernel
