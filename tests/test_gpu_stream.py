@@ -80,7 +80,7 @@ def test_layer_takes_them(fmt, T):
         assert L.stream_tile_m(fmt, T, K, E, NS, H, I) == want
     else:
         n = L.decode_max_tiles(T * (K + NS), min(E, T * K) + NS)
-        assert L.decode_stream_gate_up(fmt, T, H, I, n) == (fmt != F.FMT_BF16)
+        assert L.decode_stream_gate_up(fmt, T, H, I, n)
         assert L.decode_stream_down(fmt, H, I, n) == (fmt != F.FMT_BF16)
     perm = torch.randperm(E + NS, generator=torch.Generator().manual_seed(1))
     Wp = ExpertWeights(fmt, H, I, E, NS, *[None if t is None else t[perm.cuda()].contiguous()

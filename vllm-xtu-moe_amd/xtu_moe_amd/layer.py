@@ -697,6 +697,9 @@ def stream_i8_tile_m(T: int, K: int, E: int, H: int) -> int:
 
 
 DECODE_STREAM_MIN_ITEMS = 384
+# bytes of staged token rows (T x H) past which the decode gate/up's
+# workgroups crowd each other out of the LDS
+DECODE_STAGE_MAX_BYTES = 40 << 10
 
 
 def decode_stream_gate_up(fmt: int, T: int, H: int, I: int, max_tiles: int) -> bool:
@@ -704,27 +707,30 @@ def decode_stream_gate_up(fmt: int, T: int, H: int, I: int, max_tiles: int) -> b
     (xtu_stream_gate_up): where the decode kernel's workgroups of 16 columns
     would stage rows piecewise or take several rounds of weights
     (xtu_decode_gate_up_fast).  Measured on MI355X: DeepSeek-V3 MXFP4 T = 5 / 8
-    / 16 149 / 225 / 366 -> 96 / 139 / 233 us, FP8 T = 3 / 16 132 / 533 -> 119 /
-    433; Qwen3-Next NVFP4 T = 6 / 16 28.5 / 80 -> 23 / 43; 128-expert FP8 T = 16
+    / 16 149 / 225 / 366 -> 96 / 139 / 233 us (T = 3 / 4, past
+    DECODE_STAGE_MAX_BYTES: layer 100.2 / 128.0 -> 97.6 / 123.2), FP8 T = 3 / 16
+    132 / 533 -> 119 / 433; Qwen3-Next NVFP4 T = 6 / 16 28.5 / 80 -> 23 / 43; 128-expert FP8 T = 16
     50 -> 43.  Where the fast form holds the decode kernel is the faster one
     (Qwen3-Next NVFP4 T = 4 19.0 vs 21.8, 128-expert FP8 T = 8 27.9 vs 29.2),
     and with few work items (tiny Mixtral T = 16: 13.2 vs 13.2)."""
-    return (not _lib.call("xtu_decode_gate_up_fast", int(fmt), int(T), int(H))
+    return ((T * H * 2 > DECODE_STAGE_MAX_BYTES
+             or not _lib.call("xtu_decode_gate_up_fast", int(fmt), int(T), int(H)))
             and max_tiles * (I // 64) >= DECODE_STREAM_MIN_ITEMS)
 
 
 STREAM_DOWN_MAX_I = 1024   # decode: the down pass streams in wide items up to this K ...
-STREAM_DOWN_MIN_ITEMS = {FMT_MXFP4: 512, FMT_FP8: 512, FMT_NVFP4: 768}   # ... and this many items
+STREAM_DOWN_MIN_ITEMS = {FMT_MXFP4: 320, FMT_FP8: 512, FMT_NVFP4: 320}   # ... and this many items
 
 
 def decode_stream_down(fmt: int, H: int, I: int, max_tiles: int) -> bool:
     """Whether a decode batch's down pass takes 128-column workgroups
     (xtu_stream_down): a short K makes the decode kernel's waves short (four
     units at I = 512).  Measured on MI355X: Qwen3-Next MXFP4 T = 4 / 8 / 16
-    10.6 / 17.1 / 27.4 -> 8.4 / 10.9 / 17.0 us, NVFP4 T = 6 / 16 14.8 / 28.8 ->
-    13.4 / 22.0 (T = 4: equal, 0.4 us slower per layer),
-    128-expert FP8 (I = 768) T = 4 10.8 -> 10.2, BF16 T = 16 40.3 vs 41.9 (not
-    taken); DeepSeek-V3 (I = 2048) T = 4 41.5 vs 42.4, T = 16 equal."""
+    10.6 / 17.1 / 27.4 -> 8.4 / 10.9 / 17.0 us, whole layer T = 2 / 3 25.2 / 27.1
+    -> 20.7 / 24.7 (336 / 496 items); NVFP4 T = 3 / 4 31.9 / 35.8 -> 29.5 / 34.4;
+    128-expert FP8 (I = 768) T = 4 10.8 -> 10.2, whole layer T = 1 / 2 (128 / 256
+    items) 17.6 / 22.8 vs 18.5 / 23.0; BF16 T = 16 40.3 vs 41.9 (not taken);
+    DeepSeek-V3 (I = 2048) T = 4 41.5 vs 42.4, T = 16 equal."""
     return (fmt in STREAM_DOWN_MIN_ITEMS and I <= STREAM_DOWN_MAX_I
             and max_tiles * (H // 128) >= STREAM_DOWN_MIN_ITEMS[fmt])
 
@@ -733,6 +739,10 @@ FUSED_DOWN_ENV = "XTU_DECODE_FUSED_DOWN"
 
 
 FUSED_DOWN_MAX_EXPERTS = 24
+# MXFP4 with a short K (I <= STREAM_DOWN_MAX_I): past T = 1 scale the streaming
+# down and the combine are faster than each wave walking every expert:
+# Qwen3-Next T = 2 (21 experts) 20.7 against 25.2 us per layer
+MXFP4_NARROW_FUSED_MAX = 12
 NVFP4_NARROW_FUSED_MAX = 12   # NVFP4 at I < 1024: the fused down only at T = 1 scale
 
 
@@ -746,7 +756,8 @@ def decode_fused_down_ok(fmt: int, T: int, A: int, H: int, I: int, max_active: i
 
 
 def decode_fused_down_use(fmt: int, T: int, A: int, H: int, I: int, max_active: int,
-                          trash: int, shared_rows: int = 0, one_launch: bool = False) -> bool:
+                          trash: int, shared_rows: int = 0, one_launch: bool = False,
+                          streams: bool = False) -> bool:
     """Whether the decode path takes the fused down + combine.  Each of its
     waves walks every active expert, so it pays where few experts meet wide
     panels; measured (MI355X): faster for DeepSeek-V3 MXFP4 at T = 1, 2 (9 / 17
@@ -755,12 +766,16 @@ def decode_fused_down_use(fmt: int, T: int, A: int, H: int, I: int, max_active: 
     the whole layer runs in xtu_decode_layer) at T = 1 scale (at most 12
     experts): Qwen3-Next NVFP4 T = 1 25.3 against 26.0 us (two launches with
     the separate down and combine); as a launch of its own it was slower.
+    streams: the separate down may be the streaming one (moe_forward's "auto").
     XTU_DECODE_FUSED_DOWN=1 takes it whenever it fits, =0 never."""
     mode = os.environ.get(FUSED_DOWN_ENV, "auto")
     if mode == "0":
         return False
     if mode != "1":
         if max_active > FUSED_DOWN_MAX_EXPERTS:
+            return False
+        if (streams and int(fmt) == FMT_MXFP4 and I <= STREAM_DOWN_MAX_I
+                and max_active > MXFP4_NARROW_FUSED_MAX):
             return False
         if int(fmt) == FMT_NVFP4 and I < 1024 and (not one_launch
                                                    or max_active > NVFP4_NARROW_FUSED_MAX):
@@ -809,6 +824,11 @@ FUSED_ROUTE_ENV = "XTU_DECODE_FUSED_ROUTE"
 # DeepSeek-V3 MXFP4 T = 1 (140 MB) 49.2 vs 49.1, T = 2 (265 MB) 75.5 -> 79.8,
 # T = 4 (515 MB) 130.3 -> 131.6.
 FUSED_ROUTE_MAX_BYTES = 64 << 20
+# NVFP4's stream is bound by its dequantisation as much as by memory, and the
+# routing beside it costs registers: separate launches win from T = 3 on
+# (Qwen3-Next T = 2 / 3 / 4: 25 / 37 / 48 MB, 25.9 / 34.1 / 39.3 us in one launch
+# against 26.7 / 31.9 / 35.8)
+FUSED_ROUTE_MAX_BYTES_NVFP4 = 32 << 20
 
 
 def _w13_bytes(W) -> int:
@@ -826,7 +846,8 @@ def _route_gate_up_ok(fmt, mode, T, E, K, router, H, I, NS, gu_bytes=None) -> bo
     mode_env = os.environ.get(FUSED_ROUTE_ENV, "auto")
     if mode_env == "0":
         return False
-    if mode_env != "1" and gu_bytes is not None and gu_bytes > FUSED_ROUTE_MAX_BYTES:
+    cap = FUSED_ROUTE_MAX_BYTES_NVFP4 if int(fmt) == FMT_NVFP4 else FUSED_ROUTE_MAX_BYTES
+    if mode_env != "1" and gu_bytes is not None and gu_bytes > cap:
         return False
     n_group = 1
     if router is not None:
@@ -984,7 +1005,7 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
     split = (path == "decode" and T > 0 and NS > 0 and seg.small
              and odt in (torch.bfloat16, torch.float32)
              and decode_fused_down_use(fmt, T, seg.A, H, I, max_active, E + NS, NS * T,
-                                       one_launch=layer_ok)
+                                       one_launch=layer_ok, streams=auto)
              and (fused or _route_shared_ok(fmt, rmode, T, E, K, router, H, I, NS)))
     lim, al, be = float(swiglu_limit or 0.0), float(swiglu_alpha), float(swiglu_beta)
     if split:
@@ -993,7 +1014,8 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
     # barrier across its workgroups
     one = layer_ok and (split or (odt in (torch.bfloat16, torch.float32)
                                   and decode_fused_down_use(fmt, T, seg.A, H, I, max_active,
-                                                            E + NS, one_launch=True)))
+                                                            E + NS, one_launch=True,
+                                                            streams=auto)))
     if one:
         r = router or {}
         act = _buf("act", (max(seg.A, 1), I), torch.bfloat16, dev, st)
@@ -1088,7 +1110,8 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
                       _p(seg.tile_expert), _p(seg.tile_row0), _p(seg.n_tiles), max_dt, _p(act),
                       lim, al, be, st)
         if split or (odt in (torch.bfloat16, torch.float32)
-                     and decode_fused_down_use(fmt, T, A, H, I, max_active, E + NS)):
+                     and decode_fused_down_use(fmt, T, A, H, I, max_active, E + NS,
+                                               streams=auto)):
             # down projection and weighted combine in one pass, out written whole
             _lib.call("xtu_decode_down_combine", fmt, _p(act),
                       _p(act_sh) if split else 0, NS, T, A, H, I, _p(W.w2), _p(W.s2),
