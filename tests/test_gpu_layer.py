@@ -192,3 +192,30 @@ def test_two_streams_do_not_share_scratch(path):
     torch.cuda.synchronize()
     for a, b in zip(outs, ref):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("path", ["gemm", "auto"])
+def test_nvfp4_every_scale_code(path):
+    """One expert per finite e4m3 scale code (0, the subnormals, up to 448), one
+    row each: every row against the oracle by its own norm (bf16 act rows:
+    2^-9 per element, averaged over I)."""
+    E, H, I = 127, 256, 128
+    d = make_dense_layer(F.FMT_NVFP4, E, H, I, seed=11)
+    codes = torch.arange(E, dtype=torch.uint8)[:, None, None]
+    d["s13"], d["s2"] = codes.expand_as(d["s13"]).contiguous(), codes.expand_as(d["s2"]).contiguous()
+    d["gs13"], d["gs2"] = torch.ones_like(d["gs13"]), torch.ones_like(d["gs2"])
+    W = ExpertWeights.from_dense(F.FMT_NVFP4, d["w13"], d["s13"], d["w2"], d["s2"], d["gs13"],
+                                 d["gs2"], device="cuda")
+    ids = np.random.default_rng(3).permutation(E).astype(np.int32)[:, None].copy()
+    wts = np.ones((E, 1), np.float32)
+    x = torch.randn((E, H), generator=torch.Generator().manual_seed(12)).to(torch.bfloat16)
+    out = moe_forward(x.cuda(), torch.from_numpy(ids).cuda(), torch.from_numpy(wts).cuda(), W,
+                      path=path, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    ref = oracle_layer(F.FMT_NVFP4, dense_to_numpy(F.FMT_NVFP4, d), bf16_tensor_to_bits(x), ids, wts,
+                       E, 0, H, I).astype(np.float64)
+    o = out.cpu().numpy().astype(np.float64)
+    zero = ids[:, 0] == 0
+    assert (o[zero] == 0).all() and (ref[zero] == 0).all()
+    err = np.linalg.norm(o - ref, axis=1)[~zero] / np.linalg.norm(ref, axis=1)[~zero]
+    assert float(err.max()) <= 2.0 ** -8, (path, int(ids[~zero][err.argmax()]), float(err.max()))
