@@ -697,9 +697,15 @@ def stream_i8_tile_m(T: int, K: int, E: int, H: int) -> int:
 
 
 DECODE_STREAM_MIN_ITEMS = 384
-# bytes of staged token rows (T x H) past which the decode gate/up's
-# workgroups crowd each other out of the LDS
-DECODE_STAGE_MAX_BYTES = 40 << 10
+# Bytes of staged token rows (T x H) past which the decode gate/up's
+# workgroups crowd each other out of the LDS, for the formats of 8 and 16
+# bits: BF16 128 experts T = 14 / 16 126 / 135 us streamed against 130 / 140,
+# Qwen3-Next T = 14 137 against 143, FP8 H = 4096 T = 8 159 against 163 (layers in
+# a chain).  The 4-bit ones hold the fast form to T = 4 only and lose by it at
+# every width: DeepSeek-V3 T = 3 / 4 MXFP4 118 / 151 us streamed against 101 /
+# 128, NVFP4 142 / 176 against 120 / 149; H = 8192 T = 4 MXFP4 147 against 127,
+# H = 6144 T = 4 NVFP4 116 against 106.
+DECODE_STAGE_MAX_BYTES = {FMT_FP8: 40 << 10, FMT_BF16: 40 << 10}
 
 
 def decode_stream_gate_up(fmt: int, T: int, H: int, I: int, max_tiles: int) -> bool:
@@ -707,13 +713,13 @@ def decode_stream_gate_up(fmt: int, T: int, H: int, I: int, max_tiles: int) -> b
     (xtu_stream_gate_up): where the decode kernel's workgroups of 16 columns
     would stage rows piecewise or take several rounds of weights
     (xtu_decode_gate_up_fast).  Measured on MI355X: DeepSeek-V3 MXFP4 T = 5 / 8
-    / 16 149 / 225 / 366 -> 96 / 139 / 233 us (T = 3 / 4, past
-    DECODE_STAGE_MAX_BYTES: layer 100.2 / 128.0 -> 97.6 / 123.2), FP8 T = 3 / 16
-    132 / 533 -> 119 / 433; Qwen3-Next NVFP4 T = 6 / 16 28.5 / 80 -> 23 / 43; 128-expert FP8 T = 16
+    / 16 149 / 225 / 366 -> 96 / 139 / 233 us, FP8 T = 3 / 16 132 / 533 -> 119 /
+    433; Qwen3-Next NVFP4 T = 6 / 16 28.5 / 80 -> 23 / 43; 128-expert FP8 T = 16
     50 -> 43.  Where the fast form holds the decode kernel is the faster one
-    (Qwen3-Next NVFP4 T = 4 19.0 vs 21.8, 128-expert FP8 T = 8 27.9 vs 29.2),
-    and with few work items (tiny Mixtral T = 16: 13.2 vs 13.2)."""
-    return ((T * H * 2 > DECODE_STAGE_MAX_BYTES
+    (Qwen3-Next NVFP4 T = 4 19.0 vs 21.8, 128-expert FP8 T = 8 27.9 vs 29.2) up
+    to DECODE_STAGE_MAX_BYTES, and with few work items (tiny Mixtral T = 16:
+    13.2 vs 13.2)."""
+    return ((T * H * 2 > DECODE_STAGE_MAX_BYTES.get(int(fmt), math.inf)
              or not _lib.call("xtu_decode_gate_up_fast", int(fmt), int(T), int(H)))
             and max_tiles * (I // 64) >= DECODE_STREAM_MIN_ITEMS)
 
