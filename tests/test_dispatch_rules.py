@@ -21,3 +21,12 @@ def _gate_up_streams(fmt, T, E, NS, H, I, K):
     (FMT_BF16, 10, 2048, False), (FMT_BF16, 11, 2048, True)])
 def test_decode_gate_up_streams_past_the_fast_form(fmt, T, H, want):
     assert _gate_up_streams(fmt, T, 256, 1, H, 2048, 8) == want
+
+
+@pytest.mark.parametrize("fmt,I,want", [(FMT_MXFP4, 768, True), (FMT_MXFP4, 1024, False),
+                                        (FMT_FP8, 768, True), (FMT_FP8, 896, False),
+                                        (FMT_NVFP4, 512, True), (FMT_NVFP4, 640, False),
+                                        (FMT_BF16, 512, False)])
+def test_decode_down_streams_at_a_short_k(fmt, I, want):
+    assert L.decode_stream_down(fmt, 2048, I, 64) == want
+    assert not L.decode_stream_down(fmt, 2048, I, 16)   # 256 work items

@@ -724,7 +724,8 @@ def decode_stream_gate_up(fmt: int, T: int, H: int, I: int, max_tiles: int) -> b
             and max_tiles * (I // 64) >= DECODE_STREAM_MIN_ITEMS)
 
 
-STREAM_DOWN_MAX_I = 1024   # decode: the down pass streams in wide items up to this K ...
+# decode: the down pass streams in wide items up to this K ...
+STREAM_DOWN_MAX_I = {FMT_MXFP4: 768, FMT_FP8: 768, FMT_NVFP4: 512}
 STREAM_DOWN_MIN_ITEMS = {FMT_MXFP4: 320, FMT_FP8: 512, FMT_NVFP4: 320}   # ... and this many items
 
 
@@ -735,9 +736,15 @@ def decode_stream_down(fmt: int, H: int, I: int, max_tiles: int) -> bool:
     10.6 / 17.1 / 27.4 -> 8.4 / 10.9 / 17.0 us, whole layer T = 2 / 3 25.2 / 27.1
     -> 20.7 / 24.7 (336 / 496 items); NVFP4 T = 3 / 4 31.9 / 35.8 -> 29.5 / 34.4;
     128-expert FP8 (I = 768) T = 4 10.8 -> 10.2, whole layer T = 1 / 2 (128 / 256
-    items) 17.6 / 22.8 vs 18.5 / 23.0; BF16 T = 16 40.3 vs 41.9 (not taken);
-    DeepSeek-V3 (I = 2048) T = 4 41.5 vs 42.4, T = 16 equal."""
-    return (fmt in STREAM_DOWN_MIN_ITEMS and I <= STREAM_DOWN_MAX_I
+    items) 17.6 / 22.8 vs 18.5 / 23.0; BF16 T = 16 40.3 vs 41.9 (not taken).
+    Longer K, whole layers in a chain, the decode kernel against this one:
+    NVFP4 I = 768 (128 experts) T = 3 / 8 31.7 / 51.9 vs 33.1 / 52.9, I = 640
+    (H = 6144) T = 6 53.2 vs 53.8; MXFP4 I = 768 (H = 4096, 32 experts) T = 4 / 16
+    36.2 / 53.8 vs 35.3 / 52.6, I = 1024 (64 experts) T = 4 / 8 49.5 / 73.6 vs
+    50.6 / 76.5, (256 experts) T = 16 84.0 vs 85.8, (16 experts) 50.1 vs 48.5;
+    FP8 I = 768 (H = 4096) T = 16 68.1 vs 65.9, I = 1024 (256 experts) T = 4 / 8
+    46.6 / 71.3 vs 47.8 / 72.7."""
+    return (fmt in STREAM_DOWN_MIN_ITEMS and I <= STREAM_DOWN_MAX_I[fmt]
             and max_tiles * (H // 128) >= STREAM_DOWN_MIN_ITEMS[fmt])
 
 
@@ -745,9 +752,10 @@ FUSED_DOWN_ENV = "XTU_DECODE_FUSED_DOWN"
 
 
 FUSED_DOWN_MAX_EXPERTS = 24
-# MXFP4 with a short K (I <= STREAM_DOWN_MAX_I): past T = 1 scale the streaming
+# MXFP4 with a short K (I <= MXFP4_NARROW_MAX_I): past T = 1 scale the streaming
 # down and the combine are faster than each wave walking every expert:
 # Qwen3-Next T = 2 (21 experts) 20.7 against 25.2 us per layer
+MXFP4_NARROW_MAX_I = 1024
 MXFP4_NARROW_FUSED_MAX = 12
 NVFP4_NARROW_FUSED_MAX = 12   # NVFP4 at I < 1024: the fused down only at T = 1 scale
 
@@ -780,7 +788,7 @@ def decode_fused_down_use(fmt: int, T: int, A: int, H: int, I: int, max_active: 
     if mode != "1":
         if max_active > FUSED_DOWN_MAX_EXPERTS:
             return False
-        if (streams and int(fmt) == FMT_MXFP4 and I <= STREAM_DOWN_MAX_I
+        if (streams and int(fmt) == FMT_MXFP4 and I <= MXFP4_NARROW_MAX_I
                 and max_active > MXFP4_NARROW_FUSED_MAX):
             return False
         if int(fmt) == FMT_NVFP4 and I < 1024 and (not one_launch
