@@ -1,6 +1,7 @@
 """The layer's dispatch rules (host code only): which kernels a decode batch
 takes, at shapes on each side of a line."""
 import pytest
+import torch
 
 from xtu_moe_amd import layer as L
 from xtu_moe_amd.formats import FMT_BF16, FMT_FP8, FMT_MXFP4, FMT_NVFP4
@@ -30,3 +31,24 @@ def test_decode_gate_up_streams_past_the_fast_form(fmt, T, H, want):
 def test_decode_down_streams_at_a_short_k(fmt, I, want):
     assert L.decode_stream_down(fmt, 2048, I, 64) == want
     assert not L.decode_stream_down(fmt, 2048, I, 16)   # 256 work items
+
+
+@pytest.mark.parametrize("T,K,NS,E,H,I,fused", [
+    # 13 to 24 active experts of MXFP4 at a short K: the separate down where it
+    # writes pair order, the fused one where it cannot (K = 7; three shared)
+    (2, 8, 0, 128, 2048, 768, False), (2, 8, 1, 256, 2048, 512, False),
+    (2, 7, 3, 256, 2048, 512, True), (2, 6, 3, 256, 2048, 512, True),
+    (2, 8, 1, 256, 2048, 2048, True), (1, 10, 1, 512, 2048, 512, True)])
+def test_fused_down_leaves_only_for_the_down_in_pair_order(T, K, NS, E, H, I, fused):
+    active = min(E, T * K) + NS
+    by_pair = L.down_by_pair(K, NS, torch.bfloat16)
+    assert by_pair == (K in L.COMBINE_BY_PAIR_K and NS <= 2)
+    assert L.decode_fused_down_use(FMT_MXFP4, T, T * (K + NS), H, I, active, E + NS,
+                                   by_pair=by_pair) == fused
+
+
+def test_down_by_pair_switch(monkeypatch):
+    monkeypatch.setenv(L.DOWN_BY_PAIR_ENV, "0")
+    assert not L.down_by_pair(8, 1, torch.bfloat16)
+    monkeypatch.delenv(L.DOWN_BY_PAIR_ENV)
+    assert not L.down_by_pair(8, 1, torch.float16)

@@ -752,9 +752,14 @@ FUSED_DOWN_ENV = "XTU_DECODE_FUSED_DOWN"
 
 
 FUSED_DOWN_MAX_EXPERTS = 24
-# MXFP4 with a short K (I <= MXFP4_NARROW_MAX_I): past T = 1 scale the streaming
-# down and the combine are faster than each wave walking every expert:
-# Qwen3-Next T = 2 (21 experts) 20.7 against 25.2 us per layer
+# MXFP4 with a short K (I <= MXFP4_NARROW_MAX_I): past T = 1 scale the down in
+# pair order (streaming or not) and the combine are as fast as each wave
+# walking every expert, or faster; layers in a chain against the fused down:
+# streaming, Qwen3-Next T = 2 (21 experts) 24.1 / 26.7 us, H = 7168 I = 512 T = 2
+# 36.6 / 38.5; decode kernel, 64 experts H = 1024 I = 512 T = 2 / 3 22.8 / 26.2 and
+# 24.1 / 28.3, 256 experts I = 1024 T = 2 27.5 / 33.4, 128 experts I = 768 T = 2
+# equal, at worst (K = 6, H = 4096, I = 1024, T = 3) 36.6 / 35.9.  Not where y is
+# per sorted position: three shared experts, K = 7 / 6 26.5 / 22.6 and 23.9 / 21.8.
 MXFP4_NARROW_MAX_I = 1024
 MXFP4_NARROW_FUSED_MAX = 12
 NVFP4_NARROW_FUSED_MAX = 12   # NVFP4 at I < 1024: the fused down only at T = 1 scale
@@ -771,7 +776,7 @@ def decode_fused_down_ok(fmt: int, T: int, A: int, H: int, I: int, max_active: i
 
 def decode_fused_down_use(fmt: int, T: int, A: int, H: int, I: int, max_active: int,
                           trash: int, shared_rows: int = 0, one_launch: bool = False,
-                          streams: bool = False) -> bool:
+                          by_pair: bool = False) -> bool:
     """Whether the decode path takes the fused down + combine.  Each of its
     waves walks every active expert, so it pays where few experts meet wide
     panels; measured (MI355X): faster for DeepSeek-V3 MXFP4 at T = 1, 2 (9 / 17
@@ -780,7 +785,8 @@ def decode_fused_down_use(fmt: int, T: int, A: int, H: int, I: int, max_active: 
     the whole layer runs in xtu_decode_layer) at T = 1 scale (at most 12
     experts): Qwen3-Next NVFP4 T = 1 25.3 against 26.0 us (two launches with
     the separate down and combine); as a launch of its own it was slower.
-    streams: the separate down may be the streaming one (moe_forward's "auto").
+    by_pair: the separate down would write y in flat pair order (down_by_pair
+    under moe_forward's "auto").
     XTU_DECODE_FUSED_DOWN=1 takes it whenever it fits, =0 never."""
     mode = os.environ.get(FUSED_DOWN_ENV, "auto")
     if mode == "0":
@@ -788,7 +794,7 @@ def decode_fused_down_use(fmt: int, T: int, A: int, H: int, I: int, max_active: 
     if mode != "1":
         if max_active > FUSED_DOWN_MAX_EXPERTS:
             return False
-        if (streams and int(fmt) == FMT_MXFP4 and I <= MXFP4_NARROW_MAX_I
+        if (by_pair and int(fmt) == FMT_MXFP4 and I <= MXFP4_NARROW_MAX_I
                 and max_active > MXFP4_NARROW_FUSED_MAX):
             return False
         if int(fmt) == FMT_NVFP4 and I < 1024 and (not one_launch
@@ -804,6 +810,12 @@ SHARED_SPLIT_ENV = "XTU_DECODE_SHARED_SPLIT"
 # shared experts, and the combine issues all its loads at once.
 DOWN_BY_PAIR_ENV = "XTU_DECODE_DOWN_BY_PAIR"
 COMBINE_BY_PAIR_K = (1, 2, 4, 6, 8, 10)
+
+
+def down_by_pair(K: int, NS: int, out_dtype) -> bool:
+    """Whether the separate decode down writes y in flat pair order."""
+    return (os.environ.get(DOWN_BY_PAIR_ENV, "1") != "0" and K in COMBINE_BY_PAIR_K
+            and NS <= 2 and out_dtype in (torch.bfloat16, torch.float32))
 
 
 def _route_shared_ok(fmt, mode, T, E, K, router, H, I, NS) -> bool:
@@ -1006,6 +1018,7 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
     seg = segmentation(T, K, E, NS, bm, dev, st)
     odt = out_dtype if out is None else out.dtype
     max_active = min(E, T * K) + NS
+    by_pair = auto and down_by_pair(K, NS, odt)
     # decode with shared experts: their gate/up runs in the routing launch
     # (they need no routing), the routed gate/up leaves them out and the fused
     # down takes their rows from act_sh
@@ -1019,7 +1032,7 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
     split = (path == "decode" and T > 0 and NS > 0 and seg.small
              and odt in (torch.bfloat16, torch.float32)
              and decode_fused_down_use(fmt, T, seg.A, H, I, max_active, E + NS, NS * T,
-                                       one_launch=layer_ok, streams=auto)
+                                       one_launch=layer_ok, by_pair=by_pair)
              and (fused or _route_shared_ok(fmt, rmode, T, E, K, router, H, I, NS)))
     lim, al, be = float(swiglu_limit or 0.0), float(swiglu_alpha), float(swiglu_beta)
     if split:
@@ -1029,7 +1042,7 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
     one = layer_ok and (split or (odt in (torch.bfloat16, torch.float32)
                                   and decode_fused_down_use(fmt, T, seg.A, H, I, max_active,
                                                             E + NS, one_launch=True,
-                                                            streams=auto)))
+                                                            by_pair=by_pair)))
     if one:
         r = router or {}
         act = _buf("act", (max(seg.A, 1), I), torch.bfloat16, dev, st)
@@ -1125,7 +1138,7 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
                       lim, al, be, st)
         if split or (odt in (torch.bfloat16, torch.float32)
                      and decode_fused_down_use(fmt, T, A, H, I, max_active, E + NS,
-                                               streams=auto)):
+                                               by_pair=by_pair)):
             # down projection and weighted combine in one pass, out written whole
             _lib.call("xtu_decode_down_combine", fmt, _p(act),
                       _p(act_sh) if split else 0, NS, T, A, H, I, _p(W.w2), _p(W.s2),
@@ -1134,8 +1147,7 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
                       _p(out), int(out.dtype == torch.bfloat16), st)
             return (out, seg) if return_seg else out
         y = _buf("y", (max(A, 1), H), torch.float32, dev, st)
-        if (os.environ.get(DOWN_BY_PAIR_ENV, "1") != "0" and K in COMBINE_BY_PAIR_K
-                and NS <= 2 and out.dtype in (torch.bfloat16, torch.float32)):
+        if down_by_pair(K, NS, out.dtype):
             # y rows in flat pair order: the combine's loads need no inv first
             if auto and decode_stream_down(fmt, H, I, max_dt):
                 lo, hi = seg.tile_range_ptrs(0, E + NS)
