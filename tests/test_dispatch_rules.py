@@ -52,3 +52,12 @@ def test_down_by_pair_switch(monkeypatch):
     assert not L.down_by_pair(8, 1, torch.bfloat16)
     monkeypatch.delenv(L.DOWN_BY_PAIR_ENV)
     assert not L.down_by_pair(8, 1, torch.float16)
+
+
+@pytest.mark.parametrize("T,K,E,NS,small", [(64, 16, 1024, 0, True), (341, 3, 1024, 0, True),
+                                            (341, 3, 1025, 0, False), (2, 4, 2047, 0, False),
+                                            (2, 4, 3, 1, False), (1, 3, 3, 1, True),
+                                            (2, 17, 64, 0, False), (64, 16, 1024, 1, False)])
+def test_small_segmentation_takes_what_its_entry_takes(T, K, E, NS, small):
+    """At most 1024 experts and K <= E besides the pair and bucket limits."""
+    assert L.segmentation(T, K, E, NS, 16, "cpu", stream=0).small == small

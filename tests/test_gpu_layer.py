@@ -219,3 +219,23 @@ def test_nvfp4_every_scale_code(path):
     assert (o[zero] == 0).all() and (ref[zero] == 0).all()
     err = np.linalg.norm(o - ref, axis=1)[~zero] / np.linalg.norm(ref, axis=1)[~zero]
     assert float(err.max()) <= 2.0 ** -8, (path, int(ids[~zero][err.argmax()]), float(err.max()))
+
+
+@pytest.mark.parametrize("E,T,K", [(1025, 2, 4), (1025, 60, 4), (3, 2, 4)])
+def test_given_ids_past_the_one_launch_segmentation(E, T, K):
+    """More than 1024 experts, and more choices than experts, with ids given and
+    few pairs: the segmentation in two launches."""
+    H, I = 256, 128
+    d = make_dense_layer(F.FMT_BF16, E, H, I, seed=E)
+    W = ExpertWeights.from_dense(F.FMT_BF16, d["w13"], None, d["w2"], None, device="cuda")
+    rng = np.random.default_rng(E + T)
+    ids = rng.integers(0, E, (T, K)).astype(np.int32)
+    ids[-1, -1] = E - 1
+    wts = rng.random((T, K)).astype(np.float32) + 0.05
+    x = torch.randn((T, H), generator=torch.Generator().manual_seed(T)).to(torch.bfloat16)
+    out = moe_forward(x.cuda(), torch.from_numpy(ids).cuda(), torch.from_numpy(wts).cuda(), W,
+                      out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    ref = oracle_layer(F.FMT_BF16, dense_to_numpy(F.FMT_BF16, d), bf16_tensor_to_bits(x), ids, wts,
+                       E, 0, H, I)
+    check_close(out.cpu().numpy(), ref, bf16_out=False, what=f"E={E} T={T} K={K}")

@@ -23,6 +23,7 @@ from .formats import (FMT_BF16, FMT_FP8, FMT_INT4, FMT_MXFP4, FMT_NVFP4, INT4_GR
 DECODE_MAX_TOKENS = 16
 DECODE_TILE = 16     # rows per work slot of the decode kernels (one MFMA M tile)
 SMALL_MAX_PAIRS = 1024
+SMALL_MAX_EXPERTS = 1024
 # The one-launch router routes 4 tokens at a time in one workgroup (the tiny
 # path one wave per token); past this many tokens the multi-workgroup router
 # plus the three-launch segmentation is faster (measured: 95 us vs ~17 us for
@@ -369,7 +370,9 @@ class _Segmentation:
 
     @property
     def small(self) -> bool:
-        return self.A <= SMALL_MAX_PAIRS and self.E + self.NS + 1 <= 2048 and self.K <= 16
+        """Whether xtu_route_segment_small takes the shape (its checks)."""
+        return (self.A <= SMALL_MAX_PAIRS and self.E <= SMALL_MAX_EXPERTS
+                and self.E + self.NS + 1 <= 2048 and self.K <= min(16, self.E))
 
     def tile_range_ptrs(self, b0: int, b1: int):
         """Device pointers to expert_tile_start[b0] and [b1] (m-tile range of buckets [b0, b1))."""
