@@ -317,7 +317,7 @@ int xtu_decode_gate_up_fast(int fmt, int T, int H);
 /* The INT8 ALIGN products (xtu_i8_gemm_gate_up / _down below, bit for bit)
  * read from the MXFP4 codes and scales themselves, expanded in registers
  * (half the bytes of the expanded planes): a8 / crow from xtu_i8_quant_rows,
- * emin from xtu_i8_prepare, tiles of at most 128 rows. */
+ * emin from xtu_i8_emin, tiles of at most 128 rows. */
 hipError_t xtu_stream_i8_gate_up(const int8_t* a8, const int32_t* crow, int T,
                                  const int32_t* sorted_tok, int H, int I, const void* w13,
                                  const void* s13, const uint8_t* emin13, const int32_t* slot_map,
@@ -538,10 +538,13 @@ hipError_t xtu_mx_duo_down(const uint8_t* q, const uint8_t* sq, int H, int I, co
  * its output column unwritten (gate/up: act column n when gate row n or up
  * row n is marked) and xtu_i8_fallback computes it in fp32 -- the reference
  * sends such tiles to its fp32 path (moe_v2_packed4_w4a8.inc:1344-1366).
+ * xtu_i8_emin: emin and *dmax alone, all that xtu_stream_i8_* needs.
  * xtu_i8_quant_rows: per-row power-of-two int8 quantisation of bf16 rows.
  * The GEMMs accumulate in int32 (optionally stored to acc_out [A][N]) and
  * apply 2^(emin-128+crow) in fp32; epilogues as the bf16 GEMMs. */
 size_t xtu_i8_weight_bytes(int N, int K);
+hipError_t xtu_i8_emin(const void* s, int E, int N, int K, void* emin, int32_t* dmax,
+                       hipStream_t stream);
 hipError_t xtu_i8_prepare(const void* w, const void* s, int E, int N, int K, void* w8, void* emin,
                           int32_t* dmax, hipStream_t stream);
 hipError_t xtu_i8_quant_rows(const void* rows_bf16, int M, int K, int8_t* a8, int32_t* crow,

@@ -122,3 +122,28 @@ def test_int8_offset_guard_rows_take_fp32():
     from helpers import rel_l2
     assert rel_l2(o[tiny], ref32) < 1e-4
     assert rel_l2(ref8[tiny], ref32) < 1e-4      # the oracle restates the same guard
+
+
+@pytest.mark.parametrize("mutable", [False, True])
+def test_int8_automatic_path_keeps_no_expanded_weights(mutable):
+    """The streaming GEMMs read the codes: a layer that only takes them holds
+    emin and the fallback lists (marked rows here), not the int8 planes; the
+    same bits as the integer GEMMs over the planes, built when first asked."""
+    E, NS, H, I, K, T = 8, 1, 512, 512, 2, 200
+    d = _marked(E, NS, H, I, seed=87)
+    W0 = ExpertWeights.from_dense(F.FMT_MXFP4, d["w13"], d["s13"], d["w2"], d["s2"], n_shared=NS,
+                                  device=DEV)
+    W = ExpertWeights(F.FMT_MXFP4, H, I, E, NS, W0.w13, W0.s13, W0.w2, W0.s2, mutable=mutable)
+    rng = np.random.default_rng(88)
+    ids = torch.from_numpy(np.stack([rng.permutation(E)[:K] for _ in range(T)]).astype(np.int32))
+    wts = torch.from_numpy((rng.random((T, K)) + 0.05).astype(np.float32))
+    x = torch.randn((T, H), generator=torch.Generator().manual_seed(89)).to(torch.bfloat16)
+    args = (x.to(DEV), ids.to(DEV), wts.to(DEV), W)
+    kw = dict(int8=True, swiglu_limit=7.0, out_dtype=torch.float32)
+    a = moe_forward(*args, **kw)
+    assert W._i8 is None and W.int8_fallback_cols() is not None
+    b = moe_forward(*args, path="gemm", **kw)
+    torch.cuda.synchronize()
+    assert W._i8 is not None and torch.equal(a, b)
+    e13, e2 = W.int8_emin()
+    assert torch.equal(e13, W._i8[1]) and torch.equal(e2, W._i8[3])

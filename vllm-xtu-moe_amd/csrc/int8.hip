@@ -16,8 +16,8 @@
 // kernels compute exactly those columns in fp32 from the MXFP4 weights and
 // the bf16 activations (the fp32 path's operands).
 //
-// The shifted int8 weights are expanded once per layer (xtu_i8_prepare) into
-// the P16 panel layout with 16 int8 per chunk, next to a per-row emin; the
+// Where the integer GEMMs here run, the shifted int8 weights are expanded once
+// per layer (xtu_i8_prepare) into the P16 panel layout with 16 int8 per chunk, next to a per-row emin; the
 // GEMM then runs v_mfma_i32_32x32x32_i8 on LDS tiles with the same tile list
 // and epilogues as the bf16 grouped GEMM.  A resident layer's automatic path
 // streams the codes and expands them in registers instead (stream.hip: half
@@ -648,20 +648,26 @@ extern "C" {
 
 size_t xtu_i8_weight_bytes(int N, int K) { return (size_t)N * (size_t)K; }
 
-hipError_t xtu_i8_prepare(const void* w, const void* s, int E, int N, int K, void* w8,
-                          void* emin, int32_t* dmax, hipStream_t stream) {
+hipError_t xtu_i8_emin(const void* s, int E, int N, int K, void* emin, int32_t* dmax,
+                       hipStream_t stream) {
   // dmax must hold 0 on entry; it receives the largest b - emin over all rows
   XTU_CHECK_ARG(E > 0 && N > 0 && K > 0 && N % 16 == 0 && K % 128 == 0);
-  XTU_CHECK_ARG(w && s && w8 && emin && dmax);
+  XTU_CHECK_ARG(s && emin && dmax);
   (void)hipGetLastError();
-  const long w_es = WFmt<kMXFP4>::w_bytes(N, K), s_es = WFmt<kMXFP4>::s_bytes(N, K),
-             w8_es = (long)N * K;
-  i8_emin_kernel<<<dim3((N + 255) / 256, E), 256, 0, stream>>>((const uint8_t*)s, N, K, s_es,
-                                                               (uint8_t*)emin, dmax);
+  i8_emin_kernel<<<dim3((N + 255) / 256, E), 256, 0, stream>>>(
+      (const uint8_t*)s, N, K, WFmt<kMXFP4>::s_bytes(N, K), (uint8_t*)emin, dmax);
+  return hipPeekAtLastError();
+}
+
+hipError_t xtu_i8_prepare(const void* w, const void* s, int E, int N, int K, void* w8,
+                          void* emin, int32_t* dmax, hipStream_t stream) {
+  XTU_CHECK_ARG(w && w8);
+  const hipError_t err = xtu_i8_emin(s, E, N, K, emin, dmax, stream);
+  if (err != hipSuccess) return err;
   const long nch = (long)N * K / 32;
   i8_expand_kernel<<<dim3((unsigned)((nch + 255) / 256), E), 256, 0, stream>>>(
-      (const uint8_t*)w, (const uint8_t*)s, N, K, w_es, s_es, (const uint8_t*)emin,
-      (uint8_t*)w8, w8_es);
+      (const uint8_t*)w, (const uint8_t*)s, N, K, WFmt<kMXFP4>::w_bytes(N, K),
+      WFmt<kMXFP4>::s_bytes(N, K), (const uint8_t*)emin, (uint8_t*)w8, (long)N * K);
   return hipPeekAtLastError();
 }
 

@@ -110,6 +110,7 @@ SIGNATURES = {
     "xtu_copy_experts": (_i, [_i, _vp, _vp, _l, _vp, _l, _l, _vp]),
     "xtu_copy_2d": (_i, [_vp, _sz, _vp, _sz, _sz, _sz, _vp]),
     "xtu_i8_weight_bytes": (_sz, [_i, _i]),
+    "xtu_i8_emin": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp]),
     "xtu_i8_prepare": (_i, [_vp, _vp, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "xtu_i8_quant_rows": (_i, [_vp, _i, _i, _vp, _vp, _vp]),
     "xtu_i8_gemm_gate_up": (_i, [_vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,

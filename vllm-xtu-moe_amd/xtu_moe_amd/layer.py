@@ -96,6 +96,7 @@ class ExpertWeights:
         self.mutable = bool(mutable)
         self.slot_fp8_scales_ok = fp8_scales_ok
         self._i8 = None
+        self._i8_emin = None
         self._i8_fb = None
         self._i8_emm = None
         self._mxs = None
@@ -198,13 +199,27 @@ class ExpertWeights:
     # ---------------------------------------------------------------- INT8
     def int8_planes(self):
         """Shifted int8 weights + per-row emin for the INT8 ALIGN path (MXFP4
-        only).  Rows whose e8m0 spread exceeds 3 are marked (emin 0xFF); their
-        output columns take the fp32 fallback (int8_fallback_cols).  Cached,
-        except for mutable planes, whose contents change between calls: for
-        those each call prepares them again (and int8_fallback_cols then
-        returns that call's fallback columns)."""
+        only): (w13, emin13, w2, emin2), what the integer GEMMs over expanded
+        weights read (twice the code bytes; int8_emin is all that the
+        streaming ones need).  Rows whose e8m0 spread exceeds 3 are marked
+        (emin 0xFF); their output columns take the fp32 fallback
+        (int8_fallback_cols).  Cached, except for mutable planes, whose
+        contents change between calls: for those each call prepares them again
+        (and int8_fallback_cols then returns that call's fallback columns)."""
         if self._i8 is not None and not self.mutable:
             return self._i8
+        self._i8 = self._int8_prepare(expand=True)
+        return self._i8
+
+    def int8_emin(self):
+        """(emin13, emin2): int8_planes' per-row emin without the expanded
+        weights; cached and prepared again as those."""
+        if self._i8_emin is not None and not self.mutable:
+            return self._i8_emin
+        self._int8_prepare(expand=False)
+        return self._i8_emin
+
+    def _int8_prepare(self, expand):
         if self.fmt != FMT_MXFP4:
             raise ValueError("the INT8-activation path needs MXFP4 (e8m0) weights")
         n = self.n_slots
@@ -214,14 +229,19 @@ class ExpertWeights:
         dmax = torch.zeros(1, dtype=torch.int32, device=dev)
         emm = []
         for (w, s, N, K) in ((self.w13, self.s13, 2 * self.I, self.H), (self.w2, self.s2, self.H, self.I)):
-            w8 = torch.empty((n, N * K), dtype=torch.uint8, device=dev)
             emin = torch.empty((n, N), dtype=torch.uint8, device=dev)
-            _lib.call("xtu_i8_prepare", _p(w), _p(s), n, N, K, _p(w8), _p(emin), _p(dmax), st)
+            w8 = None
+            if expand:
+                w8 = torch.empty((n, N * K), dtype=torch.uint8, device=dev)
+                _lib.call("xtu_i8_prepare", _p(w), _p(s), n, N, K, _p(w8), _p(emin), _p(dmax), st)
+            else:
+                _lib.call("xtu_i8_emin", _p(s), n, N, K, _p(emin), _p(dmax), st)
             out += [w8, emin]
             # each slot's smallest e8m0 byte: the offset guard's weight side
             mm = torch.empty(n, dtype=torch.int32, device=dev)
             _lib.call("xtu_i8_emin_min", _p(s), n, N, K, _p(mm), st)
             emm.append(mm)
+        self._i8_emin = (out[1], out[3])
         self._i8_emm = tuple(emm)
         self._i8_fb = None
         if int(dmax.item()) > 3:   # marked rows: CSR lists of their output columns per slot
@@ -230,23 +250,22 @@ class ExpertWeights:
             m13 = (m13[:, :I] | m13[:, I:])            # column pair n: gate row n or up row n
             m2 = (out[3] == I8_MARKED).cpu()
             self._i8_fb = _csr_cols(m13, dev) + _csr_cols(m2, dev)
-        self._i8 = tuple(out)
-        return self._i8
+        return tuple(out)
 
     def int8_emin_min(self):
         """(eminmin13, eminmin2): int32 [slots], each slot's smallest e8m0 byte
         of its gate/up and down matrices (the offset guard's weight side),
-        from the same preparation as int8_planes (for mutable planes: the
+        from the same preparation as int8_emin (for mutable planes: the
         last one, as int8_fallback_cols)."""
-        if self._i8 is None:
-            self.int8_planes()
+        if self._i8_emin is None:
+            self.int8_emin()
         return self._i8_emm
 
     def int8_fallback_cols(self):
         """None, or (start13, cols13, start2, cols2): per weight slot, the
         gate/up column pairs and down columns the fp32 fallback computes."""
-        if self._i8 is None:
-            self.int8_planes()
+        if self._i8_emin is None:
+            self.int8_emin()
         return self._i8_fb
 
 
@@ -1211,7 +1230,10 @@ def expert_pass(x, seg, W: ExpertWeights, b0: int, b1: int, y, *, slot_map=None,
     act = _buf("act", (max(A, 1), I), torch.bfloat16, dev, st)
     lo, hi = seg.tile_range_ptrs(b0, b1)
     if int8:
-        w13_8, emin13, w2_8, emin2 = W.int8_planes()
+        if stream_bm:   # the codes, expanded in registers
+            emin13, emin2 = W.int8_emin()
+        else:
+            w13_8, emin13, w2_8, emin2 = W.int8_planes()
         a8x = _buf("a8x", (T, H), torch.int8, dev, st)
         crx = _buf("crx", (T,), torch.int32, dev, st)
         a8a = _buf("a8a", (max(A, 1), I), torch.int8, dev, st)
