@@ -185,6 +185,27 @@ def hook_for(cfg, W):
     return hook
 
 
+def gate_up_choice(fmt, T, E, NS, H, I, K, i8, W):
+    """(kernel, tile height, grid's tile bound) of the gate/up that moe_forward
+    runs for T tokens (its launch apart from the routing's)."""
+    from xtu_moe_amd import layer as L
+
+    A, slots = T * (K + NS), min(E, T * K) + NS
+    if T <= L.DECODE_MAX_TOKENS and not i8:
+        tiles = L.decode_max_tiles(A, slots)
+        streams = L.decode_stream_gate_up(fmt, T, H, I, tiles)
+        return ("stream_gemm_kernel" if streams else "decode_gate_up_kernel"), L.DECODE_TILE, tiles
+    bm = L.stream_i8_tile_m(T, K, E, H) if i8 else L.stream_tile_m(fmt, T, K, E, NS, H, I)
+    if bm:
+        name = "stream_gemm_kernel"
+    else:
+        bm = L.gemm_tile_m(fmt, i8, H, I, W)
+        name = ("i8_gemm_kernel" if i8 else "f8_pair_gemm_kernel" if L.fp8_pair32_use(W)
+                else "mx_pair_gemm_kernel" if L.mx_pair_kernel(fmt, H, I)
+                else "gemm8_kernel" if L.pair_gemm(fmt, H, I) else "moe_gemm_kernel")
+    return name, bm, int(L._lib.call("xtu_segment_max_tiles", T, K, E, NS, bm))
+
+
 def bench_one(args):
     """One workload; returns its JSON line (the streamed workload prints its own)."""
     import numpy as np
@@ -192,10 +213,9 @@ def bench_one(args):
 
     from xtu_moe_amd import _lib
     from xtu_moe_amd import formats as F
-    from xtu_moe_amd.layer import (_fp8pair_bufs, _mxpair_bufs, _p, _stream, fp8_pair32_use,
-                                   gemm_tile_m, int8_align_on, moe_forward, mx_act_mode,
-                                   mx_pair_kernel, mx_tri, pair_gemm, route, segmentation,
-                                   stream_i8_tile_m, stream_tile_m)
+    from xtu_moe_amd.layer import (_fp8pair_bufs, _mxpair_bufs, _p, _stream, int8_align_on,
+                                   moe_forward, mx_act_mode, mx_tri, pair_gemm, route,
+                                   segmentation)
     from xtu_moe_amd.synthetic import synth_layer
 
     cfg = WORKLOADS[args.workload]
@@ -211,7 +231,7 @@ def bench_one(args):
     t0 = time.time()
     W = synth_layer(fmt, E, NS, H, I, seed=0, device=dev)
     if cfg["int8"]:
-        W.int8_planes()
+        W.int8_emin()
     torch.cuda.synchronize()
     log(f"[bench] built {E}+{NS} experts fmt={cfg['fmt']} in {time.time() - t0:.1f}s")
     # decode: a graph of CHAIN layers with distinct weights, each layer's output
@@ -237,7 +257,7 @@ def bench_one(args):
     e_bytes13 = F.algorithmic_bytes(fmt, 2 * I, H)
     e_bytes = e_bytes13 + F.algorithmic_bytes(fmt, H, I)
     nsteps = args.warmup + args.steps
-    results = {}
+    results, gu_kernel = {}, {}   # gu_kernel: the gate/up kernel timed at each T
     for T in cfg["Ts"]:
         # INT8 activations where the reference engine's token-count gate takes them
         i8 = cfg["int8"] and int8_align_on(T, True)
@@ -385,12 +405,10 @@ def bench_one(args):
         # ---- dominant kernel alone (gate/up), cold cache, same stream
         seg = None
         gu_ms = []
-        decode = T <= 16 and not i8
-        # the kernel the layer takes: the weight-streaming GEMMs or the prefill ones
-        sbm = 0 if decode else (stream_i8_tile_m(T, K, E, H) if i8
-                                else stream_tile_m(fmt, T, K, E, NS, H, I))
-        bm = sbm or gemm_tile_m(fmt, i8, H, I, W)
-        f8q = not decode and not i8 and not sbm and fp8_pair32_use(W)
+        gu_kernel[T], bm, max_t = gate_up_choice(fmt, T, E, NS, H, I, K, i8, W)
+        decode = gu_kernel[T] == "decode_gate_up_kernel"
+        sbm = bm if gu_kernel[T] == "stream_gemm_kernel" else 0
+        f8q = gu_kernel[T] == "f8_pair_gemm_kernel"
         act = torch.empty((T * K + T * NS, I), dtype=torch.bfloat16, device=dev)
         # one untimed call first: a kernel's code object loads on its first
         # launch (the layer above may have run only other kernels)
@@ -403,17 +421,18 @@ def bench_one(args):
             if f8q:
                 f8x = _mxpair_bufs("xm", T, H, dev)
                 _lib.call("xtu_pair_quant_il", _p(x_st), T, H, *[_p(t) for t in f8x], st)
-            elif not decode and not i8 and not sbm and mx_pair_kernel(fmt, H, I):
+            elif gu_kernel[T] == "mx_pair_gemm_kernel":
                 mxk = mx_act_mode(fmt, H, I)
                 mxx = _mxpair_bufs("xm", T, H, dev)
                 s13p, _ = W.mx_pair_scales()
                 _lib.call(f"xtu_{'pair' if mxk == 'pair' else 'tri'}_quant_il", _p(x_st), T, H,
                           *[_p(t) for t in mxx], st)
-            elif not decode and not i8 and not sbm and pair_gemm(fmt, H, I):
+            elif gu_kernel[T] == "gemm8_kernel":
                 fp8x = _fp8pair_bufs("x8", T, H, dev)
                 _lib.call("xtu_fp8pair_quant", _p(x_st), T, H, *[_p(t) for t in fp8x], st)
             if i8:
-                w13_8, emin13, _, _ = W.int8_planes()
+                emin13 = W.int8_emin()[0]
+                w13_8 = None if sbm else W.int8_planes()[0]
                 a8x = torch.empty((T, H), dtype=torch.int8, device=dev)
                 crx = torch.empty(T, dtype=torch.int32, device=dev)
                 _lib.call("xtu_i8_quant_rows", _p(x_st), T, H, _p(a8x), _p(crx), st)
@@ -424,50 +443,50 @@ def bench_one(args):
             if decode:
                 _lib.call("xtu_decode_gate_up", fmt, _p(x_st), T, H, I, _p(W.w13), _p(W.s13),
                           _p(W.gs13), 0, 0, 0, _p(seg.sorted_tok), _p(seg.seg_start),
-                          _p(seg.active), 0, _p(seg.n_active), min(E, T * K) + NS, _p(act),
-                          cfg["limit"], 1.0, 0.0, st)
+                          _p(seg.tile_expert), _p(seg.tile_row0), _p(seg.n_tiles), max_t,
+                          _p(act), cfg["limit"], 1.0, 0.0, st)
             elif sbm and i8:
                 lo, hi = seg.tile_range_ptrs(0, E + NS)
                 _lib.call("xtu_stream_i8_gate_up", _p(a8x), _p(crx), T, _p(seg.sorted_tok), H, I,
                           _p(W.w13), _p(W.s13), _p(emin13), 0, _p(seg.seg_start),
-                          _p(seg.tile_expert), _p(seg.tile_row0), lo, hi, sbm, seg.max_tiles,
+                          _p(seg.tile_expert), _p(seg.tile_row0), lo, hi, sbm, max_t,
                           _p(act), cfg["limit"], 1.0, 0.0, st)
             elif sbm:
                 lo, hi = seg.tile_range_ptrs(0, E + NS)
                 _lib.call("xtu_stream_gate_up", fmt, _p(x_st), T, _p(seg.sorted_tok), H, I,
                           _p(W.w13), _p(W.s13), _p(W.gs13), 0, 0, 0, _p(seg.seg_start),
-                          _p(seg.tile_expert), _p(seg.tile_row0), lo, hi, sbm, seg.max_tiles,
+                          _p(seg.tile_expert), _p(seg.tile_row0), lo, hi, sbm, max_t,
                           _p(act), cfg["limit"], 1.0, 0.0, st)
             elif i8:
                 lo, hi = seg.tile_range_ptrs(0, E + NS)
                 _lib.call("xtu_i8_gemm_gate_up", _p(a8x), _p(crx), _p(seg.sorted_tok), H, I,
                           _p(w13_8), _p(emin13), 0, _p(seg.seg_start), _p(seg.tile_expert),
-                          _p(seg.tile_row0), lo, hi, seg.max_tiles, _p(act), 0, cfg["limit"],
+                          _p(seg.tile_row0), lo, hi, max_t, _p(act), 0, cfg["limit"],
                           1.0, 0.0, st)
             elif f8x is not None:
                 lo, hi = seg.tile_range_ptrs(0, E + NS)
                 _lib.call("xtu_f8_pair_gate_up", *[_p(t) for t in f8x], _p(seg.sorted_tok), H, I,
                           _p(W.w13), _p(W.s13), 0, 0, 0, _p(seg.seg_start), _p(seg.tile_expert),
-                          _p(seg.tile_row0), _p(seg.expert_tile_start), lo, hi, seg.max_tiles,
+                          _p(seg.tile_row0), _p(seg.expert_tile_start), lo, hi, max_t,
                           _p(act), cfg["limit"], 1.0, 0.0, st)
             elif mxx is not None:
                 lo, hi = seg.tile_range_ptrs(0, E + NS)
                 _lib.call(f"xtu_mx_{mxk}_gate_up", *[_p(t) for t in mxx], _p(seg.sorted_tok), H, I,
                           _p(W.w13), _p(s13p), 0, 0, 0, _p(seg.seg_start), _p(seg.tile_expert),
-                          _p(seg.tile_row0), _p(seg.expert_tile_start), lo, hi, seg.max_tiles,
+                          _p(seg.tile_row0), _p(seg.expert_tile_start), lo, hi, max_t,
                           _p(act), cfg["limit"], 1.0, 0.0, st)
             elif fp8x is not None:
                 lo, hi = seg.tile_range_ptrs(0, E + NS)
                 _lib.call("xtu_gemm_pair_gate_up", fmt, *[_p(t) for t in fp8x],
                           _p(seg.sorted_tok), H, I, _p(W.w13), _p(W.s13), 0, 0, 0,
                           _p(seg.seg_start), _p(seg.tile_expert), _p(seg.tile_row0),
-                          _p(seg.expert_tile_start), lo, hi, seg.max_tiles, _p(act),
+                          _p(seg.expert_tile_start), lo, hi, max_t, _p(act),
                           cfg["limit"], 1.0, 0.0, st)
             else:
                 lo, hi = seg.tile_range_ptrs(0, E + NS)
                 _lib.call("xtu_gemm_gate_up", fmt, _p(x_st), _p(seg.sorted_tok), H, I, _p(W.w13),
                           _p(W.s13), _p(W.gs13), 0, 0, 0, _p(seg.seg_start), _p(seg.tile_expert),
-                          _p(seg.tile_row0), lo, hi, seg.max_tiles, _p(act), cfg["limit"], 1.0,
+                          _p(seg.tile_row0), lo, hi, max_t, _p(act), cfg["limit"], 1.0,
                           0.0, st)
             b.record()
             torch.cuda.synchronize()
@@ -539,10 +558,9 @@ def bench_one(args):
 
     if decode_head:
         roof = dict(bound="hbm", achieved=r["gate_up_GBs"], peak=HBM_PEAK_GBS, unit="GB/s",
-                    frac=r["gate_up_GBs"] / HBM_PEAK_GBS, traffic=None,
-                    kernel="decode_gate_up_kernel")
+                    frac=r["gate_up_GBs"] / HBM_PEAK_GBS, traffic=None, kernel=gu_kernel[Th])
         if not args.no_traffic:
-            tr = measure_traffic(args.workload, Th)
+            tr = measure_traffic(args.workload, Th, kernel=gu_kernel[Th])
             if tr is not None:
                 roof["traffic"] = tr["bytes"]
                 roof["traffic_detail"] = tr
@@ -553,31 +571,29 @@ def bench_one(args):
         # a batch whose weights outweigh its arithmetic (tiny Mixtral: 128
         # tokens over 8 experts of 12.6 MB): the grouped GEMM against HBM
         roof = dict(bound="hbm", achieved=r["gate_up_GBs"], peak=HBM_PEAK_GBS, unit="GB/s",
-                    frac=r["gate_up_GBs"] / HBM_PEAK_GBS, traffic=None, kernel="moe_gemm_kernel",
+                    frac=r["gate_up_GBs"] / HBM_PEAK_GBS, traffic=None, kernel=gu_kernel[Th],
                     layer_frac=r["layer_GBs"] / HBM_PEAK_GBS)
-    elif mx_tri(fmt, H, I) and not cfg["int8"] and not decode_head:
+    elif gu_kernel[Th] == "mx_pair_gemm_kernel" and mx_tri(fmt, H, I):
         # fp6 / fp4 A (activation triples, or their first two pieces) x e2m1
         # B on the double-rate 32x32x64 MFMA: the fp6/fp4 peak; every
         # algorithmic product is three (two) MFMA products
         ach = r["gate_up_TFLOPs"]
         npc = 2.0 if mx_act_mode(fmt, H, I) == "duo" else 3.0
         roof = dict(bound="mfma", achieved=ach, peak=PEAK_TFLOPS["fp4"], unit="TFLOP/s",
-                    frac=ach / PEAK_TFLOPS["fp4"], traffic=None, kernel="mx_pair_gemm_kernel",
+                    frac=ach / PEAK_TFLOPS["fp4"], traffic=None, kernel=gu_kernel[Th],
                     activation_pieces=int(npc),
                     mfma_issue_frac=npc * ach / PEAK_TFLOPS["fp4"],
                     frac_of_fp8_peak=ach / PEAK_TFLOPS["fp8"],
                     frac_of_bf16_peak=ach / PEAK_TFLOPS["bf16"])
         prefill_traffic(roof, "mx_pair_gemm_kernel<true")
-    elif pair_gemm(fmt, H, I) and not cfg["int8"]:
+    elif gu_kernel[Th] in ("mx_pair_gemm_kernel", "f8_pair_gemm_kernel", "gemm8_kernel"):
         # scaled MFMA with an e4m3 A (FP8: e4m3 B; MXFP4: e2m1 B), which runs
         # at the fp8 rate; every algorithmic product is two MFMA products
         # (the activation's hi and lo halves)
         ach = r["gate_up_TFLOPs"]
         roof = dict(bound="mfma", achieved=ach, peak=PEAK_TFLOPS["fp8"], unit="TFLOP/s",
                     frac=ach / PEAK_TFLOPS["fp8"], traffic=None,
-                    kernel=("mx_pair_gemm_kernel" if mx_pair_kernel(fmt, H, I)
-                            else "f8_pair_gemm_kernel" if fp8_pair32_use(W)
-                            else "gemm8_kernel"),
+                    kernel=gu_kernel[Th],
                     mfma_issue_frac=2.0 * ach / PEAK_TFLOPS["fp8"],
                     frac_of_bf16_peak=ach / PEAK_TFLOPS["bf16"])
         if roof["kernel"] == "f8_pair_gemm_kernel":
@@ -588,7 +604,7 @@ def bench_one(args):
         dt = "int8" if cfg["int8"] else "bf16"
         roof = dict(bound="mfma", achieved=r["gate_up_TFLOPs"], peak=PEAK_TFLOPS[dt],
                     unit="TFLOP/s", frac=r["gate_up_TFLOPs"] / PEAK_TFLOPS[dt], traffic=None,
-                    kernel="stream_gemm_kernel",
+                    kernel=gu_kernel[Th],
                     frac_of_fp8_peak=r["gate_up_TFLOPs"] / PEAK_TFLOPS["fp8"])
 
     cpu = None
@@ -638,16 +654,15 @@ COPY_BYTES = 256 << 20   # calibration copy for the memory counters
 
 def pmc_child(args, cfg, T):
     """Run under rocprofv3 --pmc by measure_traffic: three cold-cache launches
-    of the dominant gate/up kernel at T tokens (the decode kernel for T <= 16;
-    the MXFP4 triple or FP8 pair prefill kernel otherwise, after its
-    quantiser), then one device-to-device copy of COPY_BYTES (the counter
+    of the dominant gate/up kernel at T tokens (gate_up_choice: the decode
+    kernel, the streaming GEMM, or the MXFP4 triple or FP8 pair prefill kernel
+    after its quantiser), then one device-to-device copy of COPY_BYTES (the counter
     calibration)."""
     import torch
 
     from xtu_moe_amd import _lib
     from xtu_moe_amd import formats as F
-    from xtu_moe_amd.layer import (_mxpair_bufs, _p, _stream, fp8_pair32_use, gemm_tile_m,
-                                   mx_act_mode, mx_tri, route, segmentation)
+    from xtu_moe_amd.layer import _mxpair_bufs, _p, _stream, mx_act_mode, mx_tri, route, segmentation
     from xtu_moe_amd.synthetic import synth_layer
 
     fmt = F.fmt_of(cfg["fmt"])
@@ -661,34 +676,38 @@ def pmc_child(args, cfg, T):
     lg = torch.randn((T, E), generator=gen, device=dev)
     rkw = dict(top_k=K, scoring="sigmoid", n_group=8, topk_group=4, routed_scaling_factor=2.5)
     w_, i_ = route(lg, **rkw)
-    prefill = T > 16
-    bm = gemm_tile_m(fmt, False, H, I, W) if prefill else 128
+    name, bm, max_t = gate_up_choice(fmt, T, E, NS, H, I, K, False, W)
+    prefill = name in ("mx_pair_gemm_kernel", "f8_pair_gemm_kernel")
     seg = segmentation(T, K, E, NS, bm, dev).run(i_, w_)
     act = torch.empty((T * K + T * NS, I), dtype=torch.bfloat16, device=dev)
     flush = torch.empty(256 << 20, dtype=torch.float32, device=dev)
     st = _stream()
+    if name == "mx_pair_gemm_kernel" and mx_tri(fmt, H, I):
+        kind, s13, qname = "mx_" + mx_act_mode(fmt, H, I), W.mx_pair_scales(st)[0], "xtu_tri_quant_il"
+    elif name == "f8_pair_gemm_kernel":
+        kind, s13, qname = "f8_pair", W.s13, "xtu_pair_quant_il"
+    elif name not in ("decode_gate_up_kernel", "stream_gemm_kernel"):
+        raise SystemExit("no counter child for this prefill kernel")
     if prefill:
-        if mx_tri(fmt, H, I):
-            kind, s13 = "mx_" + mx_act_mode(fmt, H, I), W.mx_pair_scales(st)[0]
-            qname = "xtu_tri_quant_il"
-        elif fp8_pair32_use(W):
-            kind, s13, qname = "f8_pair", W.s13, "xtu_pair_quant_il"
-        else:
-            raise SystemExit("no counter child for this prefill kernel")
         xq = _mxpair_bufs("xm", T, H, dev, st)
         _lib.call(qname, _p(x), T, H, *[_p(t) for t in xq], st)
-        lo, hi = seg.tile_range_ptrs(0, E + NS)
+    lo, hi = seg.tile_range_ptrs(0, E + NS)
     for _ in range(3):
         flush.add_(1.0)
         if prefill:
             _lib.call(f"xtu_{kind}_gate_up", *[_p(t) for t in xq], _p(seg.sorted_tok), H, I,
                       _p(W.w13), _p(s13), 0, 0, 0, _p(seg.seg_start), _p(seg.tile_expert),
-                      _p(seg.tile_row0), _p(seg.expert_tile_start), lo, hi, seg.max_tiles,
+                      _p(seg.tile_row0), _p(seg.expert_tile_start), lo, hi, max_t,
                       _p(act), cfg["limit"], 1.0, 0.0, st)
+        elif name == "stream_gemm_kernel":
+            _lib.call("xtu_stream_gate_up", fmt, _p(x), T, _p(seg.sorted_tok), H, I, _p(W.w13),
+                      _p(W.s13), _p(W.gs13), 0, 0, 0, _p(seg.seg_start), _p(seg.tile_expert),
+                      _p(seg.tile_row0), lo, hi, seg.bm, max_t, _p(act), cfg["limit"], 1.0, 0.0,
+                      st)
         else:
             _lib.call("xtu_decode_gate_up", fmt, _p(x), T, H, I, _p(W.w13), _p(W.s13),
                       _p(W.gs13), 0, 0, 0, _p(seg.sorted_tok), _p(seg.seg_start),
-                      _p(seg.active), 0, _p(seg.n_active), min(E, T * K) + NS, _p(act),
+                      _p(seg.tile_expert), _p(seg.tile_row0), _p(seg.n_tiles), max_t, _p(act),
                       cfg["limit"], 1.0, 0.0, st)
     torch.cuda.synchronize()
     src = torch.ones(COPY_BYTES, dtype=torch.uint8, device=dev)
@@ -699,7 +718,7 @@ def pmc_child(args, cfg, T):
     print(f"[pmc-child] distinct experts {len(torch.unique(i_)) + NS}", flush=True)
 
 
-def measure_traffic(workload, T, timeout=150, kernel="decode_gate_up"):
+def measure_traffic(workload, T, timeout=150, kernel="decode_gate_up_kernel"):
     """HBM bytes per launch of the gate/up kernel whose name contains `kernel`
     from two rocprofv3 counter runs of pmc_child (FETCH_SIZE, then WRITE_SIZE,
     in KiB per dispatch), each scaled by the same counter's reading for a

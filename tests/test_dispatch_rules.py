@@ -61,3 +61,21 @@ def test_down_by_pair_switch(monkeypatch):
 def test_small_segmentation_takes_what_its_entry_takes(T, K, E, NS, small):
     """At most 1024 experts and K <= E besides the pair and bucket limits."""
     assert L.segmentation(T, K, E, NS, 16, "cpu", stream=0).small == small
+
+
+@pytest.mark.parametrize("wl,T,i8,kernel", [
+    ("ds-v3-mxfp4-decode", 4, False, "decode_gate_up_kernel"),
+    ("ds-v3-mxfp4-decode", 8, False, "stream_gemm_kernel"),
+    ("ds-v3-mxfp4-prefill", 8192, False, "mx_pair_gemm_kernel"),
+    ("qwen3-next-int8", 8192, True, "stream_gemm_kernel"),
+    ("qwen3-next-nvfp4", 4, False, "decode_gate_up_kernel"),
+    ("mixtral-tiny-bf16", 128, False, "moe_gemm_kernel")])
+def test_bench_times_the_gate_up_the_layer_takes(wl, T, i8, kernel):
+    bench = pytest.importorskip("bench")
+    c = bench.WORKLOADS[wl]
+    fmt = {"mxfp4": FMT_MXFP4, "nvfp4": FMT_NVFP4, "bf16": FMT_BF16}[c["fmt"]]
+    name, bm, tiles = bench.gate_up_choice(fmt, T, c["E"], c["NS"], c["H"], c["I"], c["K"], i8, None)
+    assert name == kernel
+    if T <= L.DECODE_MAX_TOKENS:
+        assert (bm, tiles) == (L.DECODE_TILE, L.decode_max_tiles(
+            T * (c["K"] + c["NS"]), min(c["E"], T * c["K"]) + c["NS"]))
