@@ -195,7 +195,7 @@ def gate_up_choice(fmt, T, E, NS, H, I, K, i8, W):
         tiles = L.decode_max_tiles(A, slots)
         streams = L.decode_stream_gate_up(fmt, T, H, I, tiles)
         return ("stream_gemm_kernel" if streams else "decode_gate_up_kernel"), L.DECODE_TILE, tiles
-    bm = L.stream_i8_tile_m(T, K, E, H) if i8 else L.stream_tile_m(fmt, T, K, E, NS, H, I)
+    bm = L.stream_i8_tile_m(T, K, E, H, I) if i8 else L.stream_tile_m(fmt, T, K, E, NS, H, I)
     if bm:
         name = "stream_gemm_kernel"
     else:

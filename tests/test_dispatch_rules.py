@@ -79,3 +79,13 @@ def test_bench_times_the_gate_up_the_layer_takes(wl, T, i8, kernel):
     if T <= L.DECODE_MAX_TOKENS:
         assert (bm, tiles) == (L.DECODE_TILE, L.decode_max_tiles(
             T * (c["K"] + c["NS"]), min(c["E"], T * c["K"]) + c["NS"]))
+
+
+def test_streaming_leaves_planes_past_32_bit_offsets():
+    """One expert's gate/up plane of 2 GiB: the kernels with 64-bit plane
+    offsets keep it (2 I H bytes of FP8, I H of MXFP4 codes)."""
+    big, fits = 1 << 16, (1 << 16) - 128
+    assert L.stream_tile_m(FMT_FP8, 64, 2, 8, 0, 16384, fits) == 64
+    assert L.stream_tile_m(FMT_FP8, 64, 2, 8, 0, 16384, big) == 0
+    assert L.stream_i8_tile_m(64, 2, 8, 32768, fits) == 64
+    assert L.stream_i8_tile_m(64, 2, 8, 32768, big) == 0

@@ -18,7 +18,7 @@ import torch
 
 from . import _lib
 from .formats import (FMT_BF16, FMT_FP8, FMT_INT4, FMT_MXFP4, FMT_NVFP4, INT4_GROUPS,
-                      int4_group_of, pack_scales, pack_weight)
+                      int4_group_of, pack_scales, pack_weight, row_bytes)
 
 DECODE_MAX_TOKENS = 16
 DECODE_TILE = 16     # rows per work slot of the decode kernels (one MFMA M tile)
@@ -687,7 +687,10 @@ def stream_tile_m(fmt: int, T: int, K: int, E: int, NS: int, H: int, I: int) -> 
     XTU_FP8_PREFILL)."""
     fmt = int(fmt)
     r = T * K / E
-    if fmt not in STREAM_MAX_ROWS or r > STREAM_MAX_ROWS[fmt] or T * H * 2 >= 1 << 31:
+    if fmt not in STREAM_MAX_ROWS or r > STREAM_MAX_ROWS[fmt]:
+        return 0
+    # 32-bit offsets: the rows of x, one expert's gate/up plane (the larger one)
+    if T * H * 2 >= 1 << 31 or 2 * I * row_bytes(fmt, H) >= 1 << 31:
         return 0
     if fmt == FMT_MXFP4 and os.environ.get(MXFP4_PREFILL_ENV, MXFP4_PREFILL_DEFAULT) != "auto":
         return 0
@@ -703,7 +706,7 @@ def stream_tile_m(fmt: int, T: int, K: int, E: int, NS: int, H: int, I: int) -> 
     return bm
 
 
-def stream_i8_tile_m(T: int, K: int, E: int, H: int) -> int:
+def stream_i8_tile_m(T: int, K: int, E: int, H: int, I: int) -> int:
     """stream_tile_m for the INT8 ALIGN path (xtu_stream_i8_*, bitwise the
     same outputs): the MXFP4 codes expanded in registers are half the bytes
     of the expanded planes, at every size measured.  Whole layer on MI355X:
@@ -711,7 +714,7 @@ def stream_i8_tile_m(T: int, K: int, E: int, H: int) -> int:
     400 / 1007 us, DeepSeek-V3 T = 500 / 4096 1916 / 3888 -> 1207 / 3491.
     tiny (8 experts) T = 160 / 4000 65 / 188 -> 44 / 176."""
     r = T * K / E
-    if T * H >= 1 << 31:
+    if T * H >= 1 << 31 or 2 * I * row_bytes(FMT_MXFP4, H) >= 1 << 31:   # 32-bit offsets
         return 0
     # a decode batch (int8 forced below its token gate) has one tile per expert
     # at either height and keeps the integer GEMMs' own
@@ -1033,7 +1036,7 @@ def moe_forward(x, topk_ids, topk_weights, W: ExpertWeights, *, swiglu_limit=0.0
     # tiles as work slots (every row of a bucket, however many)
     stream_bm = 0
     if auto and path == "gemm":
-        stream_bm = (stream_i8_tile_m(T, K, E, H) if int8
+        stream_bm = (stream_i8_tile_m(T, K, E, H, I) if int8
                      else stream_tile_m(fmt, T, K, E, NS, H, I))
     bm = (DECODE_TILE if path == "decode"
           else stream_bm or gemm_tile_m(fmt, int8, W.H, W.I, W, fp8_scales_ok))
