@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 import torch
 
+import oracle
 from helpers import (bf16_tensor_to_bits, check_close, dense_to_numpy, make_dense_layer,
                      oracle_layer, random_routing)
 from xtu_moe_amd import formats as F
@@ -342,6 +343,35 @@ def test_fused_route_softmax_512_no_shared(T, monkeypatch):
     assert L._route_gate_up_ok(fmt, 0, T, E, K, router, H, I, NS)
     _same(_fr_run(monkeypatch, True, False, x, W, K, router=router),
           _fr_run(monkeypatch, False, False, x, W, K, router=router), f"softmax 512 T={T}")
+
+
+@pytest.mark.parametrize("NS,split", [(0, False), (1, False), (1, True), (2, True)])
+@pytest.mark.parametrize("fmt,T,H", [(F.FMT_MXFP4, 1, 512), (F.FMT_MXFP4, 2, 512),
+                                     (F.FMT_MXFP4, 4, 512), (F.FMT_MXFP4, 4, 4096),
+                                     (F.FMT_FP8, 6, 4096), (F.FMT_NVFP4, 2, 2048),
+                                     (F.FMT_BF16, 2, 512)])
+def test_fused_route_softmax_128(fmt, T, H, NS, split, monkeypatch):
+    """Two experts per lane (E = 128, softmax) in the gate/up launch, at every
+    count of row pieces per thread: as the separate launches, bit for bit, and
+    the oracle; ties and signed zeros among the logits."""
+    E, I, K = 128, 256, 8
+    d, W = _layer(fmt, E, NS, H, I, seed=190 + T + NS)
+    g = torch.Generator(device="cuda").manual_seed(191 + T)
+    logits = torch.randn((T, E), generator=g, device="cuda")
+    logits[::2] = torch.round(logits[::2] * 2) / 2
+    logits[0, 3::7] = -0.0
+    x = torch.randn((T, H), generator=g, device="cuda").to(torch.bfloat16)
+    router = dict(logits=logits, scoring="softmax", renormalize=True)
+    assert L._route_gate_up_ok(fmt, 0, T, E, K, router, H, I, NS)
+    a = _fr_run(monkeypatch, True, split, x, W, K, router=router)
+    _same(a, _fr_run(monkeypatch, False, split, x, W, K, router=router),
+          f"softmax 128 fmt={fmt} T={T} NS={NS}")
+    out, ids, wts, _ = a
+    rids, rwts = oracle.route_softmax_topk(logits.cpu().numpy(), K)
+    np.testing.assert_array_equal(ids.cpu().numpy(), rids)
+    np.testing.assert_array_equal(wts.cpu().numpy().view(np.uint32), rwts.view(np.uint32))
+    ref = oracle_layer(fmt, dense_to_numpy(fmt, d), bf16_tensor_to_bits(x), rids, rwts, E, NS, H, I)
+    check_close(out.cpu().numpy(), ref, bf16_out=False, what=f"softmax 128 T={T} vs oracle")
 
 
 @pytest.mark.parametrize("split", [True, False])

@@ -32,7 +32,19 @@ def _weights(fmt, E, NS, H, I, seed):
 def test_row_tile_edges(fmt, bm, H, I):
     if bm > _lib.call("xtu_stream_max_tile_m", fmt):
         pytest.skip("taller than this format's tiles")
-    print(f"stream fmt={fmt} bm={bm} H={H} I={I}", flush=True)
+    _row_tile_edges(fmt, bm, H, I, 0)
+
+
+@pytest.mark.parametrize("bm", [64, 128])
+@pytest.mark.parametrize("H,I", [(256, 128), (768, 384)])
+def test_bf16_wide_items_row_tile_edges(bm, H, I):
+    """From 512 items on BF16 takes four panels per wave in both passes (a grid
+    bound past the tiles: the surplus workgroups leave)."""
+    _row_tile_edges(F.FMT_BF16, bm, H, I, -(-512 // min(I // 128, H // 256)))
+
+
+def _row_tile_edges(fmt, bm, H, I, min_tiles):
+    print(f"stream fmt={fmt} bm={bm} H={H} I={I} min_tiles={min_tiles}", flush=True)
     E = len(ROWS)
     ids = np.repeat(np.arange(E, dtype=np.int32), ROWS)
     rng = np.random.default_rng(bm + H)
@@ -45,16 +57,17 @@ def test_row_tile_edges(fmt, bm, H, I):
     xd, idd, wd = x.cuda(), torch.from_numpy(ids).cuda(), torch.from_numpy(wts).cuda()
     seg = L.segmentation(T, 1, E, 0, bm, torch.device("cuda")).run(idd, wd)
     lo, hi = seg.tile_range_ptrs(0, E)
+    max_tiles = max(seg.max_tiles, min_tiles)
     act = torch.full((T, I), float("nan"), dtype=torch.bfloat16, device="cuda")
     _lib.call("xtu_stream_gate_up", fmt, _p(xd), T, _p(seg.sorted_tok), H, I, _p(W.w13),
               _p(W.s13), _p(W.gs13), 0, 0, 0, _p(seg.seg_start), _p(seg.tile_expert),
-              _p(seg.tile_row0), lo, hi, bm, seg.max_tiles, _p(act), 2.0, 1.0, 0.0, _stream())
+              _p(seg.tile_row0), lo, hi, bm, max_tiles, _p(act), 2.0, 1.0, 0.0, _stream())
     ys = []
     for pair_of in (0, _p(seg.sorted_pair)):
         y = torch.full((T, H), float("nan"), device="cuda")
         _lib.call("xtu_stream_down", fmt, _p(act), H, I, _p(W.w2), _p(W.s2), _p(W.gs2), 0, 0, 0,
                   _p(seg.seg_start), _p(seg.tile_expert), _p(seg.tile_row0), lo, hi, bm,
-                  seg.max_tiles, pair_of, _p(y), _stream())
+                  max_tiles, pair_of, _p(y), _stream())
         ys.append(y)
     torch.cuda.synchronize()
     assert torch.equal(ys[0][seg.inv.long()], ys[1])
