@@ -17,12 +17,13 @@
 // the bf16 activations (the fp32 path's operands).
 //
 // Where the integer GEMMs here run, the shifted int8 weights are expanded once
-// per layer (xtu_i8_prepare) into the P16 panel layout with 16 int8 per chunk, next to a per-row emin; the
-// GEMM then runs v_mfma_i32_32x32x32_i8 on LDS tiles with the same tile list
-// and epilogues as the bf16 grouped GEMM.  A resident layer's automatic path
-// streams the codes and expands them in registers instead (stream.hip: half
-// the bytes, the same sums; Qwen3-Next T = 1000 367 -> 255 us per layer); these
-// GEMMs serve streamed layers and callers that ask for the prefill kernels.
+// per layer (xtu_i8_prepare) into the P16 panel layout with 16 int8 per chunk,
+// next to a per-row emin; the GEMM then runs v_mfma_i32_32x32x32_i8 on LDS
+// tiles with the same tile list and epilogues as the bf16 grouped GEMM.  A
+// resident layer's automatic path streams the codes and expands them in
+// registers instead (stream.hip: half the bytes, the same sums, emin alone
+// prepared; Qwen3-Next T = 1000 367 -> 255 us per layer); these GEMMs serve
+// streamed layers and callers that ask for the prefill kernels.
 #include <type_traits>
 
 #include "weight_format.hpp"

@@ -718,11 +718,12 @@ enum SmallRoute : int { kTeams = 0, kLanes = 1, kWave2 = 2, kWave4 = 4, kWave8 =
 
 // One workgroup of at least A threads and NB / 2 threads.  MODE 0: softmax
 // routing, 1: grouped sigmoid routing, 2: ids/wts given.  Then the whole
-// segmentation, one pair per thread (FEW: over at most kFewNB buckets).  Latency bound (one workgroup): with
-// the pairs ranked by ballots instead of each pair scanning the pairs before
-// it, 1023 pairs over 514 buckets 36.0 -> 6.0 us; with one wave per token
-// instead of four 256-thread teams in lockstep, T = 16 grouped sigmoid over
-// 256 experts 35.5 -> 8.8 us (routing and segmentation).
+// segmentation, one pair per thread (FEW: over at most kFewNB buckets).
+// Latency bound (one workgroup): with the pairs ranked by ballots instead of
+// each pair scanning the pairs before it, 1023 pairs over 514 buckets 36.0 ->
+// 6.0 us; with one wave per token instead of four 256-thread teams in
+// lockstep, T = 16 grouped sigmoid over 256 experts 35.5 -> 8.8 us (routing
+// and segmentation).
 template <int MODE, int RT, bool FEW>
 __global__ __launch_bounds__(kSegThreads) void route_seg_small_kernel(SmallArgs a) {
   __shared__ int s_ids[kSmallMaxA];

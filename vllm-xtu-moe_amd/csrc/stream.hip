@@ -311,7 +311,8 @@ __global__ __launch_bounds__(64 * kNW, WPS) void stream_gemm_kernel(StreamArgs a
         if constexpr (I8) {
           i32x4_t bi[PW];
 #pragma unroll
-          for (int p = 0; p < PW; ++p) bi[p] = i8_expand(tab[p], w[j][p][2 * g], w[j][p][2 * g + 1]);
+          for (int p = 0; p < PW; ++p)
+            bi[p] = i8_expand(tab[p], w[j][p][2 * g], w[j][p][2 * g + 1]);
 #pragma unroll
           for (int m = 0; m < NR; ++m) {
             const i32x4_t av = *reinterpret_cast<const i32x4_t*>(ab + m * 16 * kLD + 16 * g);
@@ -320,45 +321,46 @@ __global__ __launch_bounds__(64 * kNW, WPS) void stream_gemm_kernel(StreamArgs a
               acc[m][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bi[p], acc[m][p], 0, 0, 0);
           }
         } else {
-        bf16x8_t bv[PW];
-#pragma unroll
-        for (int p = 0; p < PW; ++p) {
-          uint32_t o[4];
-          if constexpr (FMT == kMXFP4) {
-            fp4x8_to_bf16(w[j][p][g], e8m0_to_f32(sc[p].v[0] >> (8 * j)), o);
-            bv[p] = as_bf16x8(o[0], o[1], o[2], o[3]);
-          } else if constexpr (FMT == kNVFP4) {
-            const uint32_t raw = sc[p].v[j / 2] >> (16 * (j % 2) + (g < 2 ? 0 : 8));
-            fp4x8_to_bf16_mul(w[j][p][g], e4m3_to_f32(raw & 0xffu), o);
-            bv[p] = as_bf16x8(o[0], o[1], o[2], o[3]);
-          } else if constexpr (FMT == kFP8) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              const uint32_t d = w[j][p][2 * g + h];
-              o[2 * h] = __builtin_bit_cast(
-                  uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d, 1.0f, false));
-              o[2 * h + 1] = __builtin_bit_cast(
-                  uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d, 1.0f, true));
-            }
-            bv[p] = as_bf16x8(o[0], o[1], o[2], o[3]);
-          } else {
-            bv[p] = as_bf16x8(w[j][p]);
-          }
-        }
-#pragma unroll
-        for (int m = 0; m < NR; ++m) {
-          const bf16x8_t av =
-              as_bf16x8(*reinterpret_cast<const u32x4_t*>(ab + m * 16 * kLD + 16 * g));
+          bf16x8_t bv[PW];
 #pragma unroll
           for (int p = 0; p < PW; ++p) {
-            if constexpr (FMT == kFP8) {
-              const f32x4_t c0 = (j % 2 == 0 && g == 0) ? f32x4_t{0.f, 0.f, 0.f, 0.f} : part[m][p];
-              part[m][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv[p], c0, 0, 0, 0);
+            uint32_t o[4];
+            if constexpr (FMT == kMXFP4) {
+              fp4x8_to_bf16(w[j][p][g], e8m0_to_f32(sc[p].v[0] >> (8 * j)), o);
+              bv[p] = as_bf16x8(o[0], o[1], o[2], o[3]);
+            } else if constexpr (FMT == kNVFP4) {
+              const uint32_t raw = sc[p].v[j / 2] >> (16 * (j % 2) + (g < 2 ? 0 : 8));
+              fp4x8_to_bf16_mul(w[j][p][g], e4m3_to_f32(raw & 0xffu), o);
+              bv[p] = as_bf16x8(o[0], o[1], o[2], o[3]);
+            } else if constexpr (FMT == kFP8) {
+#pragma unroll
+              for (int h = 0; h < 2; ++h) {
+                const uint32_t d = w[j][p][2 * g + h];
+                o[2 * h] = __builtin_bit_cast(
+                    uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d, 1.0f, false));
+                o[2 * h + 1] = __builtin_bit_cast(
+                    uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d, 1.0f, true));
+              }
+              bv[p] = as_bf16x8(o[0], o[1], o[2], o[3]);
             } else {
-              acc[m][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv[p], acc[m][p], 0, 0, 0);
+              bv[p] = as_bf16x8(w[j][p]);
             }
           }
-        }
+#pragma unroll
+          for (int m = 0; m < NR; ++m) {
+            const bf16x8_t av =
+                as_bf16x8(*reinterpret_cast<const u32x4_t*>(ab + m * 16 * kLD + 16 * g));
+#pragma unroll
+            for (int p = 0; p < PW; ++p) {
+              if constexpr (FMT == kFP8) {
+                const f32x4_t c0 =
+                    (j % 2 == 0 && g == 0) ? f32x4_t{0.f, 0.f, 0.f, 0.f} : part[m][p];
+                part[m][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv[p], c0, 0, 0, 0);
+              } else {
+                acc[m][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv[p], acc[m][p], 0, 0, 0);
+              }
+            }
+          }
         }
       }
       if constexpr (FMT == kFP8) {
@@ -583,7 +585,8 @@ hipError_t xtu_stream_gate_up(int fmt, const void* x, int T, const int32_t* sort
   (void)hipGetLastError();
   StreamArgs a{(const uint8_t*)x, sorted_tok, (const uint8_t*)w13, (const uint8_t*)s13, gs13,
                seg_start, tile_expert, tile_row0, tile_lo, tile_hi, slot_map, act, H, I, bm,
-               (uint32_t)((long)T * H * 2), w_estride, s_estride, limit, alpha, beta, nullptr, nullptr, nullptr};
+               (uint32_t)((long)T * H * 2), w_estride, s_estride, limit, alpha, beta, nullptr,
+               nullptr, nullptr};
   switch (fmt) {
     case kMXFP4: return launch_stream<kMXFP4>(true, a, max_tiles, stream);
     case kNVFP4: return launch_stream<kNVFP4>(true, a, max_tiles, stream);

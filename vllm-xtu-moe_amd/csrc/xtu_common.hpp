@@ -47,7 +47,8 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
 // kept), so one multiply by 2^120 rebiases both, exactly and without a branch
 // (a select on e = 0 compiles to exec-mask branches, 16 of them per four
 // super-blocks of two NVFP4 panels: 1172 -> 754 instructions with the byte
-// permute of fp4x8_to_bf16_mul).
+// permute of fp4x8_to_bf16_mul).  moe_gemm_kernel is faster with the cases and
+// has its own (gemm.hip).
 __device__ __forceinline__ float e4m3_to_f32(uint32_t b) {
   const float v = __uint_as_float((b & 0x7fu) << 20) * 1.329227995784915873e+36f;
   return __uint_as_float(__float_as_uint(v) | ((b & 0x80u) << 24));

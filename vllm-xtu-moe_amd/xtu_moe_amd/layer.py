@@ -24,10 +24,10 @@ DECODE_MAX_TOKENS = 16
 DECODE_TILE = 16     # rows per work slot of the decode kernels (one MFMA M tile)
 SMALL_MAX_PAIRS = 1024
 SMALL_MAX_EXPERTS = 1024
-# The one-launch router routes 4 tokens at a time in one workgroup (the tiny
-# path one wave per token); past this many tokens the multi-workgroup router
-# plus the three-launch segmentation is faster (measured: 95 us vs ~17 us for
-# 128 tokens over 8 experts).
+# The one-launch router has one workgroup (one wave per token, or four teams);
+# past this many tokens the multi-workgroup router and the segmentation in a
+# launch of its own are faster (95 us against ~17 for 128 tokens over 8 experts
+# with the team router).
 SMALL_ROUTE_MAX_TOKENS = 16
 TINY_MAX_PAIRS = 64  # pairs one workgroup routes and segments (xtu_route_segment_small's tiny path)
 LANE_ROUTE_MAX_E, LANE_ROUTE_MAX_K = 32, 8   # softmax routed by one thread per token
@@ -661,8 +661,13 @@ def gemm_tile_m(fmt: int, int8: bool = False, H: int = 0, I: int = 0, W=None,
 # r = 6 / 25 / 44 / 50 985 / 1213 / 1622 / 1797 vs 1205 / 1420 / 1683 / 1780 us,
 # Qwen3-Next r = 49 334 vs 414; FP8 DeepSeek-V3 r = 31 / 37 2147 / 2303 vs 2244 /
 # 2356, 128 experts r = 50 / 62 164 / 200 vs 183 / 205; BF16 128 experts r = 62 /
-# 100 / 125 248 / 294 / 364 vs 276 / 319 / 354; NVFP4 Qwen3-Next r = 21 / 80 /
-# 160 at every size (289 / 563 / 1074 vs 431 / 662 / 1220).
+# 100 / 125 248 / 294 / 364 vs 276 / 319 / 354; NVFP4 at every size measured:
+# Qwen3-Next r = 21 / 80 / 160 289 / 563 / 1074 vs 431 / 662 / 1220, DeepSeek-V3 r = 32 /
+# 64 / 128 1727 / 2680 / 4327 vs 2517 / 3175 / 4965, 8 experts (H = 4096, I = 14336) r =
+# 64 / 256 / 1024 385 / 936 / 3263 vs 460 / 1073 / 3606, (H = 1024, I = 2048) r = 32 / 256 /
+# 2048 43 / 86 / 313 vs 54 / 92 / 342, 32 experts r = 256 / 1024 665 / 2410 vs 771 / 2554.
+# FP8 over few experts r = 4 / 16 / 32 30 / 32 / 38 vs 54 / 55 / 57 (8, H = 1024) and 233 /
+# 240 / 270 vs 356 / 359 / 381 (8, H = 4096).
 STREAM_MAX_ROWS = {FMT_MXFP4: 46.0, FMT_FP8: 40.0, FMT_NVFP4: math.inf, FMT_BF16: 110.0}
 # Tile heights.  Up to SHORT rows per expert 16-row tiles (their LDS stage and
 # registers let four workgroups share a CU; a second tile of an expert reads
@@ -675,7 +680,7 @@ STREAM_SHORT_ROWS = {FMT_MXFP4: 5.0, FMT_NVFP4: 10.0}
 STREAM_TALL_ROWS = {FMT_NVFP4: 66.0, FMT_BF16: 0.0}
 STREAM_I8_TALL_ROWS = 66.0   # int8 activations: r = 59 / 80 446 / 526 vs 400 / 587 us
 # BF16 work items (128 columns) below which the prefill kernels' narrow items
-# for small batches fill the chip better: tiny Mixtral T = 128 (176 items) 36
+# for small batches fill the chip better: tiny Mixtral T = 128 (160 items) 36
 # vs 41 us.  The other formats have no such items: tiny MXFP4 58 vs 40.
 STREAM_BF16_MIN_ITEMS = 384
 
@@ -878,7 +883,8 @@ FUSED_ROUTE_MAX_BYTES = 64 << 20
 # NVFP4's stream is bound by its dequantisation as much as by memory, and the
 # routing beside it costs registers: separate launches win from T = 3 on
 # (Qwen3-Next T = 2 / 3 / 4: 25 / 37 / 48 MB, 25.9 / 34.1 / 39.3 us in one launch
-# against 26.7 / 31.9 / 35.8)
+# against 26.7 / 31.9 / 35.8; 128 experts T = 3 / 4: 42 / 56 MB, 35.2 / 38.8 against
+# 32.8 / 35.7)
 FUSED_ROUTE_MAX_BYTES_NVFP4 = 32 << 20
 
 
