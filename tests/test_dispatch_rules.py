@@ -17,9 +17,11 @@ def _gate_up_streams(fmt, T, E, NS, H, I, K):
     # however many bytes of rows it stages
     (FMT_MXFP4, 3, 7168, False), (FMT_MXFP4, 4, 7168, False), (FMT_MXFP4, 5, 7168, True),
     (FMT_NVFP4, 3, 7168, False), (FMT_NVFP4, 4, 8192, False), (FMT_NVFP4, 5, 7168, True),
-    # FP8: no fast form at H = 7168; at 4096 up to five staged rows
-    (FMT_FP8, 3, 7168, True), (FMT_FP8, 5, 4096, False), (FMT_FP8, 6, 4096, True),
-    (FMT_BF16, 10, 2048, False), (FMT_BF16, 11, 2048, True)])
+    # FP8: no fast form at H = 7168; at 4096 up to T = 8
+    (FMT_FP8, 3, 7168, True), (FMT_FP8, 8, 4096, False), (FMT_FP8, 9, 4096, True),
+    # BF16: past 40 KB of rows at H = 2048, and where K is not whole rounds
+    (FMT_BF16, 10, 2048, False), (FMT_BF16, 11, 2048, True), (FMT_BF16, 3, 4096, False),
+    (FMT_BF16, 16, 8192, False), (FMT_BF16, 3, 5120, True), (FMT_BF16, 5, 7168, True)])
 def test_decode_gate_up_streams_past_the_fast_form(fmt, T, H, want):
     assert _gate_up_streams(fmt, T, 256, 1, H, 2048, 8) == want
 

@@ -727,15 +727,23 @@ def stream_i8_tile_m(T: int, K: int, E: int, H: int, I: int) -> int:
 
 
 DECODE_STREAM_MIN_ITEMS = 384
-# Bytes of staged token rows (T x H) past which the decode gate/up's
-# workgroups crowd each other out of the LDS, for the formats of 8 and 16
-# bits: BF16 128 experts T = 14 / 16 126 / 135 us streamed against 130 / 140,
-# Qwen3-Next T = 14 137 against 143, FP8 H = 4096 T = 8 159 against 163 (layers in
-# a chain).  The 4-bit ones hold the fast form to T = 4 only and lose by it at
-# every width: DeepSeek-V3 T = 3 / 4 MXFP4 118 / 151 us streamed against 101 /
-# 128, NVFP4 142 / 176 against 120 / 149; H = 8192 T = 4 MXFP4 147 against 127,
-# H = 6144 T = 4 NVFP4 116 against 106.
-DECODE_STAGE_MAX_BYTES = {FMT_FP8: 40 << 10, FMT_BF16: 40 << 10}
+# BF16: bytes of staged token rows (T x H) past which the fast form's
+# workgroups crowd each other out of the LDS (layers in a chain: 128 experts
+# T = 14 / 16 126 / 134 us streamed against 130 / 140, Qwen3-Next T = 14 137 against
+# 143).  FP8 gains and loses as much by it (H = 4096 T = 6 / 8: 32 experts 99.8 / 110.9
+# against 97.0 / 110.6, 8 experts 225.8 / 234.7 against 221.7 / 228.3, 128 experts
+# 139.0 / 165.7 against 138.2 / 168.5), and 4-bit weights, whose fast form ends at
+# T = 4, lose at every width: DeepSeek-V3 T = 3 / 4 MXFP4 118 / 151 us streamed
+# against 101 / 128, NVFP4 142 / 176 against 120 / 149; H = 8192 T = 4 MXFP4 147 against
+# 127, H = 6144 T = 4 NVFP4 116 against 106.
+BF16_STAGE_MAX_BYTES = 40 << 10
+# BF16 rows that the decode kernel's four wave pairs walk in whole rounds of
+# four 128-k units stay with it past the fast form: H = 4096 32 experts T = 3 / 8
+# 112 / 193 us against 120 / 198 streamed, 128 experts 147 / 303 against 160 / 316,
+# H = 6144 150 / 247 against 166 / 260, H = 8192 64 experts 359 / 671 against 368 /
+# 691 (at worst, 8 experts T = 16, 4.7% the other way).  A partial last round (H =
+# 5120: T = 3 / 10 165 / 421 against 159 / 409; 7168 T = 5 558 against 546) streams.
+BF16_ROUND_H = 2048
 
 
 def decode_stream_gate_up(fmt: int, T: int, H: int, I: int, max_tiles: int) -> bool:
@@ -746,12 +754,14 @@ def decode_stream_gate_up(fmt: int, T: int, H: int, I: int, max_tiles: int) -> b
     / 16 149 / 225 / 366 -> 96 / 139 / 233 us, FP8 T = 3 / 16 132 / 533 -> 119 /
     433; Qwen3-Next NVFP4 T = 6 / 16 28.5 / 80 -> 23 / 43; 128-expert FP8 T = 16
     50 -> 43.  Where the fast form holds the decode kernel is the faster one
-    (Qwen3-Next NVFP4 T = 4 19.0 vs 21.8, 128-expert FP8 T = 8 27.9 vs 29.2) up
-    to DECODE_STAGE_MAX_BYTES, and with few work items (tiny Mixtral T = 16:
-    13.2 vs 13.2)."""
-    return ((T * H * 2 > DECODE_STAGE_MAX_BYTES.get(int(fmt), math.inf)
-             or not _lib.call("xtu_decode_gate_up_fast", int(fmt), int(T), int(H)))
-            and max_tiles * (I // 64) >= DECODE_STREAM_MIN_ITEMS)
+    (Qwen3-Next NVFP4 T = 4 19.0 vs 21.8, 128-expert FP8 T = 8 27.9 vs 29.2), as
+    with few work items (tiny Mixtral T = 16: 13.2 vs 13.2); BF16 by its rows
+    (BF16_STAGE_MAX_BYTES, BF16_ROUND_H)."""
+    if max_tiles * (I // 64) < DECODE_STREAM_MIN_ITEMS:
+        return False
+    if _lib.call("xtu_decode_gate_up_fast", int(fmt), int(T), int(H)):
+        return fmt == FMT_BF16 and T * H * 2 > BF16_STAGE_MAX_BYTES
+    return fmt != FMT_BF16 or H % BF16_ROUND_H != 0
 
 
 # decode: the down pass streams in wide items up to this K ...
