@@ -153,6 +153,16 @@ def test_fused_small_route_segment_bit_exact(T, E, K, NS, mode):
     assert int(seg.n_tiles.item()) == ets[-1]
 
 
+@pytest.mark.parametrize("T,E,K,NS,mode", [(16, 16, 4, 1, 0), (16, 17, 4, 1, 0), (128, 32, 4, 1, 0),
+                                           (3, 60, 4, 0, 0), (16, 62, 4, 1, 0), (5, 16, 4, 1, 1),
+                                           (5, 24, 4, 1, 1), (200, 16, 4, 1, 2),
+                                           (200, 17, 4, 1, 2), (170, 60, 4, 2, 2)])
+def test_few_bucket_line_bit_exact(T, E, K, NS, mode):
+    """Each side of the line between one ballot per bucket and the count table
+    (18 buckets), with every router that meets it."""
+    test_fused_small_route_segment_bit_exact(T, E, K, NS, mode)
+
+
 @pytest.mark.parametrize("T,K,E,NS", [(64, 16, 1024, 0), (93, 10, 512, 1), (341, 3, 2047, 0),
                                       (1, 1, 1, 0), (205, 4, 6, 1)])
 def test_small_segmentation_table_edges(T, K, E, NS):

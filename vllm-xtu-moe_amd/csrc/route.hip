@@ -578,7 +578,13 @@ constexpr int kSmallMaxNB = 2048;
 static_assert(kSmallMaxA <= kSegThreads && kSmallMaxNB <= 2 * kSegThreads,
               "one pair and two buckets per thread");
 
-constexpr int kFewNB = 64;   // bucket count of the ballot segmentation
+// Buckets of the ballot segmentation, at most: its ballots are one per bucket,
+// the count table's one per bit.  Routing and segmentation in one launch,
+// ballots against the table: 17 buckets grouped sigmoid T = 1 / 8 6.1 / 12.1 us
+// against 6.4 / 13.0, given ids 256 pairs 3.66 / 3.71; 25 buckets 6.9 / 13.5
+// against 6.6 / 13.7, 4.2 / 3.5; 61 buckets (softmax, K = 4) 8.6 / 15.5 against
+// 6.4 / 12.7, 6.4 / 3.7.
+constexpr int kFewNB = 18;
 
 struct FewSmem {
   int wc[kFewNB][kSegWaves];   // pairs of bucket v in wave q
