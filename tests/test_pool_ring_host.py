@@ -170,6 +170,40 @@ def test_slot_planes_size_what_is_derived_from_them():
     assert "self.n_experts" not in src
 
 
+def test_int8_preparation_publishes_whole(monkeypatch):
+    """Another thread's view while a layer prepares its INT8 state: nothing of
+    it before the lists of marked rows are there, and the lists of the first
+    preparation while the expanded planes are built."""
+    import ctypes
+
+    from xtu_moe_amd import formats as F
+    from xtu_moe_amd import layer as L
+    H, I, E = 256, 128, 3
+    mk = lambda N, K: torch.zeros((E, N * F.row_bytes(F.FMT_MXFP4, K)), dtype=torch.uint8)
+    sc = lambda N, K: torch.zeros((E, F.scale_bytes(F.FMT_MXFP4, N, K)), dtype=torch.uint8)
+    W = L.ExpertWeights(F.FMT_MXFP4, H, I, E, 0, mk(2 * I, H), sc(2 * I, H), mk(H, I), sc(H, I))
+    seen = []
+
+    def call(name, *a):
+        seen.append((name, W._i8_emin is None, W._i8_fb is None))
+        if name in ("xtu_i8_emin", "xtu_i8_prepare"):
+            emin, dmax = a[-3], a[-2]
+            ctypes.memset(emin, 0xFF, 1)                      # row 0 of slot 0 marked
+            ctypes.c_int32.from_address(dmax).value = 5
+        return 0
+
+    csr = L._csr_cols
+    monkeypatch.setattr(L._lib, "call", call)
+    monkeypatch.setattr(L, "_stream", lambda stream=None: 0)
+    monkeypatch.setattr(L, "_csr_cols", lambda m, d: (call("lists"), csr(m, d))[1])
+    W.int8_emin()
+    assert W.int8_fallback_cols() is not None
+    assert all(e and f for _, e, f in seen), seen
+    seen.clear()
+    W.int8_planes()
+    assert seen and not any(e or f for _, e, f in seen), seen
+
+
 def test_pitched_copy_refuses_bad_sizes_before_any_copy():
     """copy_hostbuf_to_device_2d returns 0 for zero or negative heights,
     widths and pitches and for spans past the host buffer, without queuing a

@@ -241,15 +241,16 @@ class ExpertWeights:
             mm = torch.empty(n, dtype=torch.int32, device=dev)
             _lib.call("xtu_i8_emin_min", _p(s), n, N, K, _p(mm), st)
             emm.append(mm)
-        self._i8_emin = (out[1], out[3])
-        self._i8_emm = tuple(emm)
-        self._i8_fb = None
+        fb = None
         if int(dmax.item()) > 3:   # marked rows: CSR lists of their output columns per slot
             I = self.I
             m13 = (out[1] == I8_MARKED).cpu()
             m13 = (m13[:, :I] | m13[:, I:])            # column pair n: gate row n or up row n
             m2 = (out[3] == I8_MARKED).cpu()
-            self._i8_fb = _csr_cols(m13, dev) + _csr_cols(m2, dev)
+            fb = _csr_cols(m13, dev) + _csr_cols(m2, dev)
+        # emin last: a thread that sees it reads lists that belong to it
+        self._i8_emm, self._i8_fb = tuple(emm), fb
+        self._i8_emin = (out[1], out[3])
         return tuple(out)
 
     def int8_emin_min(self):
